@@ -6,10 +6,11 @@
 // (one program per (batch, q_head), serial scan).
 //
 // Here the key rows [memory slots ; window ring rows] of every
-// (batch, kv_head) are split into segments of 256 rows.  A workgroup (4
+// (batch, kv_head) are split into segments of 256 rows (128 or 64 where that
+// leaves compute units idle: decode_rows_per_wave).  A workgroup (4
 // waves) owns one segment of one kv row and serves every query head of that
 // kv head it is launched for (the GQA group shares each K/V read).  A wave
-// reads 64 rows with D/8 lanes per row, i.e. 4 (D=128) or 8 (D=64) whole
+// reads 64 (32, 16) rows with D/8 lanes per row, i.e. 4 (D=128) or 8 (D=64) whole
 // rows per 16-byte-per-lane load: each load instruction covers 1 KiB of
 // contiguous HBM.  Scores, the wave softmax and the PV accumulation are in
 // fp32; the 4 waves merge (max, sum, acc) through LDS, and a second kernel
@@ -24,9 +25,7 @@
 namespace kvm {
 namespace {
 
-constexpr int kRowsPerWave = 64;
 constexpr int kWaves = 4;
-constexpr int kSegRows = kRowsPerWave * kWaves;
 constexpr float kLog2e = 1.4426950408889634f;
 
 // Non-temporal 16-byte load: every K/V row is read once per step, and the
@@ -38,7 +37,8 @@ __device__ __forceinline__ uint4 ld_stream16(const uint16_t *p) {
   return make_uint4(x[0], x[1], x[2], x[3]);
 }
 
-template <int D, int GQ>
+// RW: key rows per wave (64, 32 or 16).
+template <int D, int GQ, int RW>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(GQ == 1 ? 3 : 2))) void k_decode_partial(
     kvm_layer L, const uint16_t *__restrict__ q, int64_t q_sb, int64_t q_sh,
     const uint16_t *__restrict__ sk, const uint16_t *__restrict__ sv,
@@ -49,7 +49,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(GQ == 1 ? 3
     uint16_t *ring_k_out, uint16_t *ring_v_out, uint16_t *ring_g_out) {
   constexpr int G = D / 8;             // lanes per key row
   constexpr int RPS = 64 / G;          // rows per wave step
-  constexpr int STEPS = kRowsPerWave / RPS;
+  constexpr int STEPS = RW / RPS;
+  constexpr int kSegRows = RW * kWaves;
   __shared__ float sm_m[kWaves][GQ], sm_l[kWaves][GQ];
   __shared__ float sm_acc[kWaves][GQ][D];
 
@@ -77,7 +78,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(GQ == 1 ? 3
     tf[j] = static_cast<const float *>(L.front_temp)[hq0 + j];
   }
 
-  const int r0 = seg * kSegRows + wave * kRowsPerWave;
+  const int r0 = seg * kSegRows + wave * RW;
   const uint16_t *skrow = sk + int64_t(row) * cap * D;
   const uint16_t *svrow = sv + int64_t(row) * cap * D;
   const uint16_t *rkrow = rk + int64_t(row) * ring_cap * D;
@@ -219,8 +220,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(GQ == 1 ? 3
   }
 }
 
-// Merge the segments of one (batch, q_head) in segment order.
-template <int D>
+// Merge the segments of one (batch, q_head) in segment order.  NS: segments
+// loaded at once (8 or 16, the smaller that holds them all: a call of few
+// rows pays for the loads it predicates off).
+template <int D, int NS>
 __global__ __launch_bounds__(D) void k_decode_combine(
     int Hq, int nseg, const float *__restrict__ part_acc,
     const float *__restrict__ part_ml, uint16_t *__restrict__ out,
@@ -231,21 +234,20 @@ __global__ __launch_bounds__(D) void k_decode_combine(
   const float *ml = part_ml + int64_t(pid) * nseg * 2;
   const float *acc = part_acc + int64_t(pid) * nseg * D + d;
   float M = -INFINITY, a = 0.f, l = 0.f;
-  constexpr int kMaxSeg = 16;
-  if (nseg <= kMaxSeg) {
+  if (nseg <= NS) {
     // Every partial loaded at once (one memory round trip), then the same
     // arithmetic in the same segment order as the loop below.
-    float m[kMaxSeg], sl[kMaxSeg], x[kMaxSeg];
+    float m[NS], sl[NS], x[NS];
 #pragma unroll
-    for (int s = 0; s < kMaxSeg; ++s) {
+    for (int s = 0; s < NS; ++s) {
       m[s] = s < nseg ? ml[2 * s] : -INFINITY;
       sl[s] = s < nseg ? ml[2 * s + 1] : 0.f;
       x[s] = s < nseg ? acc[s * D] : 0.f;
     }
 #pragma unroll
-    for (int s = 0; s < kMaxSeg; ++s) M = fmaxf(M, m[s]);
+    for (int s = 0; s < NS; ++s) M = fmaxf(M, m[s]);
 #pragma unroll
-    for (int s = 0; s < kMaxSeg; ++s) {
+    for (int s = 0; s < NS; ++s) {
       if (s < nseg) {
         const float f = (m[s] == -INFINITY) ? 0.f : exp2f(m[s] - M);
         a += x[s] * f;
@@ -264,7 +266,7 @@ __global__ __launch_bounds__(D) void k_decode_combine(
   out[b * o_sb + h * o_sh + d] = uint16_t(f2bf(a / l));
 }
 
-template <int D, int GQ>
+template <int D, int GQ, int RW>
 hipError_t launch_partial(const kvm_layer &L, const void *q, int64_t q_sb,
                           int64_t q_sh, const kvm_state &st, int64_t active,
                           const void *ring_k, const void *ring_v,
@@ -275,7 +277,7 @@ hipError_t launch_partial(const kvm_layer &L, const void *q, int64_t q_sb,
   const int group = int(L.q_heads / L.kv_heads);
   dim3 grid(unsigned(nseg), unsigned(L.batch * L.kv_heads),
             unsigned(group / GQ));
-  hipLaunchKernelGGL((k_decode_partial<D, GQ>), grid, dim3(256), 0, stream, L,
+  hipLaunchKernelGGL((k_decode_partial<D, GQ, RW>), grid, dim3(256), 0, stream, L,
                      static_cast<const uint16_t *>(q), q_sb, q_sh,
                      static_cast<const uint16_t *>(st.s_k_attn),
                      static_cast<const uint16_t *>(st.s_v_attn), st.capacity,
@@ -286,7 +288,7 @@ hipError_t launch_partial(const kvm_layer &L, const void *q, int64_t q_sb,
   return hipGetLastError();
 }
 
-template <int D>
+template <int D, int RW>
 hipError_t launch_partial_d(const kvm_layer &L, const void *q, int64_t q_sb,
                             int64_t q_sh, const kvm_state &st, int64_t active,
                             const void *ring_k, const void *ring_v,
@@ -294,26 +296,75 @@ hipError_t launch_partial_d(const kvm_layer &L, const void *q, int64_t q_sb,
                             int64_t recent_len, int nseg, float *pacc,
                             float *pml, const int32_t *ctl, int pending, const kvm_seq &fresh,
                             uint16_t *rkw, uint16_t *rvw, uint16_t *rgw, hipStream_t stream) {
-  const int64_t group = L.q_heads / L.kv_heads;
+  // Query heads per workgroup: as many as share the key rows (4, 2, 1), but
+  // fewer where that would leave compute units idle (two workgroups each):
+  // one head of 64 key rows after another is a chain, and the rows read again
+  // come from the caches.  B 1, 32 heads over 8, 768 rows of 128: 9.3 us with
+  // four heads per workgroup, 7.7 with one.  Each head's arithmetic is the same.
+  const int64_t group = L.q_heads / L.kv_heads, wgs = L.batch * L.kv_heads * nseg;
+  int64_t gq = group % 4 == 0 ? 4 : group % 2 == 0 ? 2 : 1;
+  while (gq > 1 && wgs * (group / gq) < 512) gq /= 2;
 #define KVM_PARTIAL(GQ)                                                      \
-  launch_partial<D, GQ>(L, q, q_sb, q_sh, st, active, ring_k, ring_v,       \
-                        ring_cap, ring_start, recent_len, nseg, pacc, pml, \
-                        ctl, pending, fresh, rkw, rvw, rgw, stream)
-  if (group % 4 == 0) return KVM_PARTIAL(4);
-  if (group % 2 == 0) return KVM_PARTIAL(2);
+  launch_partial<D, GQ, RW>(L, q, q_sb, q_sh, st, active, ring_k, ring_v,   \
+                            ring_cap, ring_start, recent_len, nseg, pacc,   \
+                            pml, ctl, pending, fresh, rkw, rvw, rgw, stream)
+  if (gq == 4) return KVM_PARTIAL(4);
+  if (gq == 2) return KVM_PARTIAL(2);
   return KVM_PARTIAL(1);
 #undef KVM_PARTIAL
 }
 
-}  // namespace
-
-int64_t decode_segments(int64_t rows_total) {
-  return (rows_total + kSegRows - 1) / kSegRows;
+template <int D>
+void launch_combine(const kvm_layer &L, int nseg, const float *pacc, const float *pml, void *out, int64_t o_sb,
+                    int64_t o_sh, hipStream_t stream) {
+#define KVM_COMBINE(NS)                                                                                   \
+  hipLaunchKernelGGL((k_decode_combine<D, NS>), dim3(unsigned(L.batch * L.q_heads)), dim3(D), 0, stream,  \
+                     int(L.q_heads), nseg, pacc, pml, static_cast<uint16_t *>(out), o_sb, o_sh)
+  if (nseg <= 8)
+    KVM_COMBINE(8);
+  else
+    KVM_COMBINE(16);
+#undef KVM_COMBINE
 }
 
+}  // namespace
+
+namespace {
+int64_t segments(int64_t rows_total, int rw) { return (rows_total + rw * kWaves - 1) / (rw * kWaves); }
+int64_t partial_bytes(const kvm_layer &L, int64_t nseg) { return L.batch * L.q_heads * nseg * (L.head_dim + 2) * 4; }
+
+// Key rows per wave for a cache of `max_rows` rows (memory slots + window).
+// 64 fill the memory pipeline best where the launch has workgroups to spare
+// (B 64, 32 heads, 1536 rows: 233 us a step).  With few workgroups a step is
+// the latency of one wave's rows, and shorter segments win: D 128, 768 rows,
+// one launch pair, in us with 64 / 32 / 16 rows per wave:
+//   B 4, 6 heads (72 workgroups of 256 rows)     10.9 / 8.8 / 7.7
+//   B 8, 32 heads over 8 (192)                   16.5 / 14.4 / 13.2
+//   B 16, 32 heads over 8 (384)                  22.4 / 18.0 / 17.6
+//   B 8, 32 heads (768)                          17.8 / 15.3 / 15.1
+//   B 4, 32 heads of 64, 1536 rows (768)         12.5 / 11.7 / 13.2
+// At most 16 segments, which the combine kernel loads at once (32 cost it
+// 1.2 us more: B 1, 32 heads, 2048 rows 12.4 us with 16 rows per wave, 10.7
+// with 32), and only where
+// the caller's workspace holds their partials (kvm_decode_workspace_bytes
+// asks for those of 256-row segments, the least that a call needs).
+// The rule reads the cache's capacity, not the live rows, so that an eager
+// and a captured step on one workspace add in the same order.
+int decode_rows_per_wave(const kvm_layer &L, int64_t max_rows, int64_t workspace_bytes) {
+  const int64_t group = L.q_heads / L.kv_heads;
+  const int64_t gq = group % 4 == 0 ? 4 : group % 2 == 0 ? 2 : 1;
+  const int64_t wgs = L.batch * L.kv_heads * (group / gq) * segments(max_rows, 64);
+  const auto fits = [&](int rw) {
+    return segments(max_rows, rw) <= 16 && partial_bytes(L, segments(max_rows, rw)) <= workspace_bytes;
+  };
+  if (wgs <= 256 && fits(16)) return 16;
+  if (wgs <= 1024 && fits(32)) return 32;
+  return 64;
+}
+}  // namespace
+
 int64_t decode_workspace_bytes(const kvm_layer &L, int64_t max_rows) {
-  const int64_t nseg = decode_segments(max_rows < 1 ? 1 : max_rows);
-  return L.batch * L.q_heads * nseg * (L.head_dim + 2) * 4;
+  return partial_bytes(L, segments(max_rows < 1 ? 1 : max_rows, 64));
 }
 
 // ---------------------------------------------------------------------------
@@ -353,7 +404,7 @@ hipError_t launch_decode(const kvm_layer &L, const void *q, int64_t q_sb,
                          const void *ring_k, const void *ring_v,
                          int64_t ring_cap, int64_t ring_start,
                          int64_t recent_len, void *out, int64_t o_sb,
-                         int64_t o_sh, void *workspace, hipStream_t stream,
+                         int64_t o_sh, void *workspace, int64_t workspace_bytes, hipStream_t stream,
                          const int32_t *ctl, int pending, int64_t max_rows,
                          const kvm_seq *fresh, void *ring_gate) {
   // Host counters: segments for the rows present; device counters: for
@@ -366,28 +417,25 @@ hipError_t launch_decode(const kvm_layer &L, const void *q, int64_t q_sb,
   uint16_t *rk = static_cast<uint16_t *>(const_cast<void *>(ring_k));
   uint16_t *rv = static_cast<uint16_t *>(const_cast<void *>(ring_v));
   uint16_t *rg = static_cast<uint16_t *>(ring_gate);
-  const int nseg = int(decode_segments(ctl ? max_rows : active + recent_len));
+  const int rw = decode_rows_per_wave(L, st.capacity + ring_cap, workspace_bytes);
+  const int nseg = int(segments(ctl ? max_rows : active + recent_len, rw));
   const int64_t npid = L.batch * L.q_heads;
   float *pacc = static_cast<float *>(workspace);
   float *pml = pacc + npid * nseg * L.head_dim;
   hipError_t e;
+#define KVM_PARTIAL_D(D, RW)                                                                                    \
+  launch_partial_d<D, RW>(L, q, q_sb, q_sh, st, active, ring_k, ring_v, ring_cap, ring_start, recent_len, nseg, \
+                          pacc, pml, ctl, pending, fr, rk, rv, rg, stream)
   if (L.head_dim == 128)
-    e = launch_partial_d<128>(L, q, q_sb, q_sh, st, active, ring_k, ring_v,
-                              ring_cap, ring_start, recent_len, nseg, pacc,
-                              pml, ctl, pending, fr, rk, rv, rg, stream);
+    e = rw == 64 ? KVM_PARTIAL_D(128, 64) : rw == 32 ? KVM_PARTIAL_D(128, 32) : KVM_PARTIAL_D(128, 16);
   else
-    e = launch_partial_d<64>(L, q, q_sb, q_sh, st, active, ring_k, ring_v,
-                             ring_cap, ring_start, recent_len, nseg, pacc, pml,
-                             ctl, pending, fr, rk, rv, rg, stream);
+    e = rw == 64 ? KVM_PARTIAL_D(64, 64) : rw == 32 ? KVM_PARTIAL_D(64, 32) : KVM_PARTIAL_D(64, 16);
+#undef KVM_PARTIAL_D
   if (e != hipSuccess) return e;
   if (L.head_dim == 128)
-    hipLaunchKernelGGL(k_decode_combine<128>, dim3(unsigned(npid)), dim3(128),
-                       0, stream, int(L.q_heads), nseg, pacc, pml,
-                       static_cast<uint16_t *>(out), o_sb, o_sh);
+    launch_combine<128>(L, nseg, pacc, pml, out, o_sb, o_sh, stream);
   else
-    hipLaunchKernelGGL(k_decode_combine<64>, dim3(unsigned(npid)), dim3(64), 0,
-                       stream, int(L.q_heads), nseg, pacc, pml,
-                       static_cast<uint16_t *>(out), o_sb, o_sh);
+    launch_combine<64>(L, nseg, pacc, pml, out, o_sb, o_sh, stream);
   return hipGetLastError();
 }
 
