@@ -299,21 +299,30 @@ __global__ __launch_bounds__(256) void k_attn_bwd_delta(const uint16_t *dout, in
   if (ok && part == 0) delta[r] = a;
 }
 
-// Per-head temperature gradients: partials summed in a fixed order
-// (batch, chunk, tile).
-__global__ void k_attn_bwd_temps(const float *tpart, int B, int Hq, int n_chunks, int qtiles,
-                                 float *d_state, float *d_front) {
-  const int hq = blockIdx.x * blockDim.x + threadIdx.x;
-  if (hq >= Hq) return;
+// Per-head temperature gradients: one workgroup per query head, its partials
+// summed in a fixed order (strided per thread, then a tree).  One thread per
+// head reading them in series took 45 us at 8 x 6 heads of 64 tiles.
+__global__ __launch_bounds__(256) void k_attn_bwd_temps(const float *tpart, int B, int Hq, int tiles, float *d_state,
+                                                        float *d_front) {
+  __shared__ float red[4][2];
+  const int hq = blockIdx.x, tid = threadIdx.x;
   float a = 0.f, f = 0.f;
-  for (int b = 0; b < B; ++b)
-    for (int w = 0; w < n_chunks * qtiles; ++w) {
-      const int64_t wg = int64_t(b * Hq + hq) * n_chunks * qtiles + w;
-      a += tpart[wg * 2];
-      f += tpart[wg * 2 + 1];
-    }
-  d_state[hq] = a;
-  d_front[hq] = f;
+  for (int i = tid; i < B * tiles; i += 256) {
+    const float *p = tpart + (int64_t(i / tiles * Hq + hq) * tiles + i % tiles) * 2;
+    a += p[0];
+    f += p[1];
+  }
+  a = wave_sum(a);
+  f = wave_sum(f);
+  if ((tid & 63) == 0) {
+    red[tid >> 6][0] = a;
+    red[tid >> 6][1] = f;
+  }
+  __syncthreads();
+  if (tid == 0) {
+    d_state[hq] = (red[0][0] + red[1][0]) + (red[2][0] + red[3][0]);
+    d_front[hq] = (red[0][1] + red[1][1]) + (red[2][1] + red[3][1]);
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -571,8 +580,8 @@ hipError_t launch_bwd_d(const kvm_layer &L, const BwdArgs &a, const ChunkTable &
                      stream, L, a, qtiles, table, tpart);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(k_attn_bwd_temps, dim3(unsigned((L.q_heads + 63) / 64)), dim3(64), 0, stream, tpart,
-                     int(L.batch), int(L.q_heads), n_chunks, qtiles, a.d_state_temp, a.d_front_temp);
+  hipLaunchKernelGGL(k_attn_bwd_temps, dim3(unsigned(L.q_heads)), dim3(256), 0, stream, tpart, int(L.batch),
+                     int(L.q_heads), n_chunks * qtiles, a.d_state_temp, a.d_front_temp);
   if ((e = hipGetLastError()) != hipSuccess) return e;
   const int wblocks = int((a.T + BKW - 1) / BKW);
   hipLaunchKernelGGL((k_attn_bwd_dkdv<D, false>), dim3(unsigned(wblocks * rows)), dim3(NTB), 0, stream, L, a,
