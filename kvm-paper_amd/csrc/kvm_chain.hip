@@ -69,7 +69,7 @@ __device__ unsigned long long g_chain_ts[2][128][16];
       else if (blockIdx.x == 8 * (GM - 1)) g_chain_ts[1][p][k] = wall_clock64();          \
     }                                                                                    \
   } while (0)
-// The appending chain's marks: member 0 of group 0, update i of the launch.
+// The other chains' marks: workgroup 0, update i of the launch.
 #define KVM_TS_A(k)                                                                      \
   do {                                                                                   \
     if (threadIdx.x == 0 && blockIdx.x == 0 && i < 128) g_chain_ts[0][i][k] = wall_clock64(); \
@@ -1539,6 +1539,392 @@ __global__ __launch_bounds__(kChainThreads) void k_chain_fixed(
   }
 }
 
+// ---------------------------------------------------------------------------
+// The chain without appends when there are rows for every compute unit: one
+// workgroup per row, no exchange.  The slot-owner kernel above spends most of
+// an update on the latency of its exchange (8.3 us at 32 slots and 32 tokens
+// per member, C 256, 256 slots), and runs 8 launches of 32 rows for 256 rows;
+// here a row's work is done in one place and every launch is full: 32.1 us per
+// update of 256 rows against 74.4.  Bound by VALU issue (the LayerNorms and
+// sums of C tokens and S slots): prep 4.2, route 8.8 (its key fragments from
+// LDS at 64 B per clock as much), lists 3.2, keys 7.4, values 1.7 + 6.9 us.
+// 16 waves of 128 registers: with 8 waves of 256 the phases but the route
+// were slower (34.8 us).
+//
+// LDS holds the attention keys of every slot and one update's token rows
+// (merge keys, then, once every slot has summed its keys, merge values in the
+// same place); the sums s_k / s_v live in registers for the whole launch,
+// packed bf16, a slot's row in the D/8 lanes that refresh it.  One update:
+//   prep     merge keys of the C tokens (raw rows loaded during the update
+//            before) into LDS; the raw values are fetched behind it
+//   route    MFMA, waves = token groups of 32 x slot groups; a token's best
+//            (score, slot) of each slot group through LDS
+//   lists    the tokens of each slot in token order (ballots, prefix sums)
+//   keys     fp32 sums in token order, LayerNorm, own_k and snapshot rows
+//   values   gated value rows into LDS, sums, value rows of the snapshot
+// The same arithmetic, in the same order, as the kernels above.
+constexpr int kRowThreads = 1024;
+constexpr int kRowWaves = kRowThreads / 64;
+constexpr int kRowPasses = 4;  // slot (and token) rows per thread
+constexpr int kRowTiles = 2;   // 16-token tiles per wave in the route
+
+template <int D>
+struct RowMax {  // slots, and tokens per update, that LDS and the registers hold
+  static constexpr int value = kRowPasses * (kRowThreads / (D / 8));
+};
+
+template <int D>
+__global__ __launch_bounds__(kRowThreads) void k_chain_row(
+    kvm_layer L, kvm_seq src, int n_tok, kvm_state st, SnapRing snaps, ChainList list, int32_t *route_log,
+    int32_t *append_log, int64_t log_stride) {
+  constexpr int GL = D / 8;
+  constexpr int STR = D + 8;
+  constexpr int KS = D / 32;
+  constexpr int RPP = kRowThreads / GL;  // rows per pass
+  constexpr int NP = kRowPasses;
+  constexpr int MAX = RowMax<D>::value;
+  __shared__ __attribute__((aligned(16))) uint16_t own_k[MAX * STR];  // attention keys
+  __shared__ __attribute__((aligned(16))) uint16_t tok[MAX * STR];    // merge keys, then merge values
+  constexpr int TT = kRowTiles;
+  constexpr int LW = MAX / 64;  // waves whose threads have a token in the lists
+  // Route keys [slot group][token] (kRowWaves * 16 TT of them), then each wave's slot counts.
+  __shared__ __attribute__((aligned(16)))
+  uint64_t scratch[kRowWaves * 16 * TT > LW * MAX / 4 ? kRowWaves * 16 * TT : LW * MAX / 4];
+  __shared__ uint16_t sorted[MAX], off[MAX], cnt[MAX];
+  __shared__ int wtot[kRowWaves];
+  __shared__ int tok_lds[kChainMax];
+  __shared__ float own_vl[MAX];
+  __shared__ float ln_w[D], ln_b[D];
+  uint16_t *const wsc = reinterpret_cast<uint16_t *>(scratch);  // [LW][MAX]
+
+  const int tid = threadIdx.x, lane = tid & 63, part = tid % GL, sub = tid / GL;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int row = blockIdx.x;
+  const int b = row / int(L.kv_heads), h = row % int(L.kv_heads);
+  const int S = list.state_before[0];  // no appends: constant over the batch
+  const int protect = min(int(L.sink_len), S);
+  const int nblk = (S + 15) >> 4;
+  const int64_t srow = int64_t(row) * st.capacity;
+  const uint16_t *k_row = static_cast<const uint16_t *>(src.k) + b * src.k_sb + h * src.k_sh;
+  const uint16_t *v_row = static_cast<const uint16_t *>(src.v) + b * src.v_sb + h * src.v_sh;
+  const uint16_t *g_row = static_cast<const uint16_t *>(src.gate) + b * src.g_sb + h * src.g_sh;
+  uint16_t *s_k = static_cast<uint16_t *>(st.s_k), *s_v = static_cast<uint16_t *>(st.s_v);
+  uint16_t *s_ka = static_cast<uint16_t *>(st.s_k_attn), *s_va = static_cast<uint16_t *>(st.s_v_attn);
+
+  for (int d = tid; d < D; d += kRowThreads) {
+    ln_w[d] = static_cast<const float *>(L.ln_weight)[d];
+    ln_b[d] = static_cast<const float *>(L.ln_bias)[d];
+  }
+  for (int i = tid; i < list.count; i += kRowThreads) tok_lds[i] = list.tok_begin[i];
+  // Sums of slot p * RPP + sub in registers; attention keys and vlen in LDS.
+  uint4 sk[NP], sv[NP];
+  {
+    const AttnRows a0 = snap_at(snaps, list.u0);
+#pragma unroll
+    for (int p = 0; p < NP; ++p) {
+      const int j = p * RPP + sub;
+      sk[p] = sv[p] = make_uint4(0, 0, 0, 0);
+      if (j < S) {
+        sk[p] = *reinterpret_cast<const uint4 *>(s_k + (srow + j) * D + part * 8);
+        sv[p] = *reinterpret_cast<const uint4 *>(s_v + (srow + j) * D + part * 8);
+        *reinterpret_cast<uint4 *>(&own_k[j * STR + part * 8]) =
+            *reinterpret_cast<const uint4 *>(a0.k + (int64_t(row) * a0.cap + j) * D + part * 8);
+        if (part == 0) own_vl[j] = static_cast<const float *>(st.s_vlen)[srow + j];
+      }
+    }
+  }
+  __syncthreads();
+
+  // Raw rows of update i: token p * RPP + sub of the thread's pass p, keys or
+  // values, and the tokens' gates.
+  uint4 raw[NP];
+  uint16_t rg[NP];
+  auto load_keys = [&](int i) __attribute__((always_inline)) {
+    const int64_t tb = tok_lds[i];
+#pragma unroll
+    for (int p = 0; p < NP; ++p) {
+      const int t = p * RPP + sub;
+      if (p * RPP < n_tok) {
+        const int64_t tt = tb + (t < n_tok ? t : 0);
+        raw[p] = ld_stream16(k_row + tt * src.k_st + part * 8);
+        rg[p] = g_row[tt * src.g_st];
+      }
+    }
+  };
+  // Token groups of 16 TT (a power of two of them) x slot groups fill the waves.
+  int ntg = 1;
+  while (ntg * (16 * TT) < n_tok) ntg <<= 1;
+  const int nsg = kRowWaves / ntg, tg = wave % ntg, sg = wave / ntg;
+
+  load_keys(0);
+  for (int i = 0; i < list.count; ++i) {
+    const int64_t u = int64_t(list.u0) + i;
+    KVM_TS_A(0);
+    // ---- prep (model/kvm_mixer.py:120-129, model/kvm_triton_mixer.py:429-446)
+#pragma unroll
+    for (int p = 0; p < NP; ++p) {
+      if (p * RPP < n_tok) {
+        const int t = p * RPP + sub;
+        float k[8];
+        unpack8(raw[p], k);
+        prep_key<D>(k, part, L, ln_w, ln_b);
+        const float g = bf2f(rg[p]);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) k[e] = L.gate_keys ? k[e] * g : k[e];
+        *reinterpret_cast<uint4 *>(&tok[t * STR + part * 8]) = pack8(k);
+        __builtin_amdgcn_sched_barrier(0);  // one pass at a time (register pressure)
+      }
+    }
+    __syncthreads();
+
+    KVM_TS_A(1);
+    // ---- route (model/kvm_fp32_routing_reference.py:30-34)
+    if (tg * (16 * TT) < n_tok) {
+      uint4 bx[TT][KS];
+#pragma unroll
+      for (int tt = 0; tt < TT; ++tt)
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks)
+          bx[tt][ks] = *reinterpret_cast<const uint4 *>(
+              &tok[(tg * (16 * TT) + tt * 16 + (lane & 15)) * STR + ks * 32 + (lane >> 4) * 8]);
+      float best[TT];
+      int bidx[TT];
+#pragma unroll
+      for (int tt = 0; tt < TT; ++tt) {
+        best[tt] = -INFINITY;
+        bidx[tt] = -1;
+      }
+      for (int blk = sg; blk < nblk; blk += nsg) {
+        const int jb = blk * 16;
+        uint4 a[KS];
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks)
+          a[ks] = *reinterpret_cast<const uint4 *>(&own_k[(jb + (lane & 15)) * STR + ks * 32 + (lane >> 4) * 8]);
+        f32x4 accs[TT];
+#pragma unroll
+        for (int tt = 0; tt < TT; ++tt) accs[tt] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+          for (int tt = 0; tt < TT; ++tt)
+            accs[tt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(a[ks]), as_bf16x8(bx[tt][ks]), accs[tt], 0,
+                                                               0, 0);
+        const int j0 = jb + (lane >> 4) * 4;
+        const bool masked = jb < protect || jb + 16 > S;
+#pragma unroll
+        for (int tt = 0; tt < TT; ++tt) {
+          f32x4 acc = accs[tt];
+          if (masked) {  // sink slots and slots past S never win
+#pragma unroll
+            for (int x = 0; x < 4; ++x) acc[x] = (j0 + x >= protect) & (j0 + x < S) ? acc[x] : -INFINITY;
+          }
+          // The lane's four slots as a tree (the earlier keeps ties), then
+          // against the running maximum: the first maximum in slot order.
+          const bool t1 = acc[1] > acc[0], t3 = acc[3] > acc[2];
+          const float v01 = t1 ? acc[1] : acc[0], v23 = t3 ? acc[3] : acc[2];
+          const int i01 = t1 ? 1 : 0, i23 = t3 ? 3 : 2;
+          const bool th = v23 > v01;
+          const float vh = th ? v23 : v01;
+          const bool take = vh > best[tt];
+          best[tt] = take ? vh : best[tt];
+          bidx[tt] = take ? j0 + (th ? i23 : i01) : bidx[tt];
+        }
+      }
+#pragma unroll
+      for (int tt = 0; tt < TT; ++tt) {
+        uint64_t key = bidx[tt] >= 0 ? route_key(best[tt], bidx[tt]) : 0;
+#pragma unroll
+        for (int r = 0; r < 2; ++r) {
+          const uint32_t hi = uint32_t(key >> 32), lo = uint32_t(key);
+          const uint64_t other = r == 0 ? (uint64_t(xor16_lane(hi, lane)) << 32) | xor16_lane(lo, lane)
+                                        : (uint64_t(xor32_lane(hi, lane)) << 32) | xor32_lane(lo, lane);
+          key = other > key ? other : key;
+        }
+        if (lane < 16) scratch[(sg * ntg + tg) * (16 * TT) + tt * 16 + lane] = key;
+      }
+    }
+    __syncthreads();
+
+    KVM_TS_A(2);
+    {  // the raw values, in flight through the lists and the keys
+      __builtin_amdgcn_sched_barrier(0);
+      const int64_t tb = tok_lds[i];
+#pragma unroll
+      for (int p = 0; p < NP; ++p) {
+        const int t = p * RPP + sub;
+        if (p * RPP < n_tok) raw[p] = ld_stream16(v_row + (tb + (t < n_tok ? t : 0)) * src.v_st + part * 8);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    // ---- lists: thread t has token t.
+    uint64_t key = 0;
+    if (tid < n_tok)
+      for (int x = 0; x < nsg; ++x) {
+        const uint64_t o = scratch[x * (ntg * 16 * TT) + tid];
+        key = o > key ? o : key;
+      }
+    const int slot = route_key_slot(key);
+    if (tid < n_tok) {
+      const int64_t lo = u * log_stride + int64_t(row) * n_tok + tid;
+      if (route_log) route_log[lo] = slot;
+      if (append_log) append_log[lo] = 0;
+    }
+    __syncthreads();  // the route keys have been read; their place takes the counts
+    const bool has = slot >= 0;
+    uint64_t eq = __ballot(has);
+    if (wave < LW)
+#pragma unroll
+      for (int x = 0; x < MAX; x += 64) wsc[wave * MAX + x + lane] = 0;
+#pragma unroll
+    for (int bit = 0; (1 << bit) < MAX; ++bit) {
+      const uint64_t m = __ballot(has && ((slot >> bit) & 1));
+      eq &= ((slot >> bit) & 1) ? m : ~m;
+    }
+    const int rank = int(__builtin_amdgcn_mbcnt_hi(uint32_t(eq >> 32), __builtin_amdgcn_mbcnt_lo(uint32_t(eq), 0u)));
+    if (has && rank == 0) wsc[wave * MAX + slot] = uint16_t(__popcll(eq));
+    __syncthreads();
+    // Exclusive prefix: over the waves of each slot's counts (in place), then over the slots.
+    int tot = 0;
+    if (tid < MAX)
+#pragma unroll
+      for (int w = 0; w < LW; ++w) {
+        const int c = wsc[w * MAX + tid];
+        wsc[w * MAX + tid] = uint16_t(tot);
+        tot += c;
+      }
+    int incl = tot;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int y = __shfl_up(incl, o);
+      if (lane >= o) incl += y;
+    }
+    if (lane == 63) wtot[wave] = incl;
+    __syncthreads();
+    {
+      int base = incl - tot;
+#pragma unroll
+      for (int w = 0; w < LW; ++w) base += w < wave ? wtot[w] : 0;
+      if (tid < MAX) {
+        off[tid] = uint16_t(base);
+        cnt[tid] = uint16_t(tot);
+      }
+    }
+    __syncthreads();
+    if (has) sorted[off[slot] + wsc[wave * MAX + slot] + rank] = uint16_t(tid);
+    __syncthreads();
+
+    KVM_TS_A(3);
+    // Sum of the staged rows of slot j's tokens, in token order; whether there are any.
+    auto sum_rows = [&](int j, float (&x)[8]) __attribute__((always_inline)) {
+      const int n = j < S ? cnt[j] : 0, o = n > 0 ? off[j] : 0;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) x[e] = 0.f;
+      int e0 = 0;
+      for (; e0 + 4 <= n; e0 += 4) {  // four rows' reads in flight
+        uint4 r[4];
+#pragma unroll
+        for (int w = 0; w < 4; ++w)
+          r[w] = *reinterpret_cast<const uint4 *>(&tok[int(sorted[o + e0 + w]) * STR + part * 8]);
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+          float f[8];
+          unpack8(r[w], f);
+#pragma unroll
+          for (int e = 0; e < 8; ++e) x[e] += f[e];
+        }
+      }
+      for (; e0 < n; ++e0) {
+        float f[8];
+        unpack8(*reinterpret_cast<const uint4 *>(&tok[int(sorted[o + e0]) * STR + part * 8]), f);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) x[e] += f[e];
+      }
+      return n > 0;
+    };
+    const AttnRows nxt = snap_at(snaps, u + 1);
+    const __amdgpu_buffer_rsrc_t nk = l2_rsrc(nxt.k + int64_t(row) * nxt.cap * D, int64_t(S) * D * 2);
+    const __amdgpu_buffer_rsrc_t nv = l2_rsrc(nxt.v + int64_t(row) * nxt.cap * D, int64_t(S) * D * 2);
+    const bool fin = i + 1 == list.count && list.final_rows != 0;
+
+    // ---- keys (model/kvm_mixer.py:329-335): state = bf16(state + bf16(sum)),
+    // LayerNorm.  Rows past S lie past the snapshot's resource and are not stored.
+#pragma unroll
+    for (int p = 0; p < NP; ++p) {
+      if (p * RPP < S) {
+        const int j = p * RPP + sub;
+        float x[8];
+        const bool any = sum_rows(j, x);
+        uint4 kk;
+        if (__any(any)) {
+          float k[8];
+          unpack8(sk[p], k);
+          if (any) {
+            round_pack8(x);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) k[e] += x[e];
+            sk[p] = round_pack8(k);
+          }
+          layer_norm8<D>(k, part, ln_w, ln_b, float(L.ln_eps));
+          kk = pack8(k);
+          if (j < S) *reinterpret_cast<uint4 *>(&own_k[j * STR + part * 8]) = kk;
+        } else {  // no slot of this wave's pass changed
+          kk = *reinterpret_cast<const uint4 *>(&own_k[j * STR + part * 8]);
+        }
+        st16<kPolicyNT>(nk, uint32_t((j * D + part * 8) * 2), kk);
+        if (fin && j < S) *reinterpret_cast<uint4 *>(s_ka + (srow + j) * D + part * 8) = kk;
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    __syncthreads();  // every wave has read the merge keys
+    KVM_TS_A(4);
+    // ---- values
+#pragma unroll
+    for (int p = 0; p < NP; ++p) {
+      if (p * RPP < n_tok) {
+        float v[8];
+        unpack8(raw[p], v);
+        const float g = bf2f(rg[p]);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] = L.gate_values ? v[e] * g : v[e];
+        *reinterpret_cast<uint4 *>(&tok[(p * RPP + sub) * STR + part * 8]) = pack8(v);
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    if (i + 1 < list.count) load_keys(i + 1);
+    __syncthreads();
+    KVM_TS_A(5);
+#pragma unroll
+    for (int p = 0; p < NP; ++p) {
+      if (p * RPP < S) {
+        const int j = p * RPP + sub;
+        float x[8], v[8];
+        const bool any = sum_rows(j, x);
+        unpack8(sv[p], v);
+        if (any) {
+          round_pack8(x);
+#pragma unroll
+          for (int e = 0; e < 8; ++e) v[e] += x[e];
+          sv[p] = round_pack8(v);
+        }
+        const uint4 vv = attn_value8_packed<D>(v, j < S ? own_vl[j] : 0.f);
+        st16<kPolicyNT>(nv, uint32_t((j * D + part * 8) * 2), vv);
+        if (fin && j < S) *reinterpret_cast<uint4 *>(s_va + (srow + j) * D + part * 8) = vv;
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    __syncthreads();  // every wave has read the merge values
+    KVM_TS_A(6);
+  }
+#pragma unroll
+  for (int p = 0; p < NP; ++p) {
+    const int j = p * RPP + sub;
+    if (j < S) {
+      *reinterpret_cast<uint4 *>(s_k + (srow + j) * D + part * 8) = sk[p];
+      *reinterpret_cast<uint4 *>(s_v + (srow + j) * D + part * 8) = sv[p];
+    }
+  }
+}
+
 __global__ __launch_bounds__(256) void k_fill_u32(unsigned *p, int64_t n, unsigned v) {
   const int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x;
   if (i < n) p[i] = v;
@@ -1558,16 +1944,16 @@ bool chain_plan(const kvm_layer &L, int64_t n_tok, int64_t max_slots, ChainPlan 
   const int64_t groups = (rows + 7) / 8 * 8;
   int G = groups * 16 <= limit ? 16 : 8;
   // More rows than one launch keeps resident: consecutive launches over
-  // batches of rows (a multiple of 8, one group per XCD each).
-  const int64_t batch_groups = std::min<int64_t>(groups, limit / G / 8 * 8);
+  // batches of rows (launch_chain).
   const int64_t tpw = ((n_tok + G - 1) / G + 15) / 16 * 16;
-  if (tpw > kChainTok || batch_groups < 8 || n_tok < 1) return false;
+  if (tpw > kChainTok || limit / G < 8 || n_tok < 1) return false;
   p->fixed = false;
   p->G = G;
+  p->limit = int(limit);
+  p->rows = int(rows);
+  p->head_dim = int(L.head_dim);
   p->tpw = int(tpw);
   p->spm_max = int((max_slots + G - 1) / G);
-  p->row_batch = int(batch_groups);
-  p->workgroups = int(batch_groups * G);
   // ints of the lists, then the append selection's 8-byte keys (a power of
   // two of them) after one int of alignment padding.
   int64_t npow = 1;
@@ -1578,14 +1964,52 @@ bool chain_plan(const kvm_layer &L, int64_t n_tok, int64_t max_slots, ChainPlan 
   return true;
 }
 
+namespace {
+// Members per row of a chain without appends over S slots (1: k_chain_row),
+// or 0 when none fits.  Up to 16 rows: 16 members (chain_plan).  Above, more
+// members make an update shorter but fewer rows fit a launch, so the choice
+// is the least of launches x time per update.  Measured at D 128, C = S, us
+// per update for all rows, with 8 / 4 / 1 members:
+//   C 256   48 rows 18.5 / 12.1 / 28.0    96 rows 27.8 / 23.7 / 29.4
+//          128 rows 37.1 / 24.5 / 30.1   256 rows 74.4 / 48.4 / 32.8
+//   C 128   64 rows 13.7 /  7.7 / 15.3   128 rows 27.6 / 15.4 / 15.6
+//   C  64  128 rows 24.5 / 12.5 /  8.6
+// (C 512: one launch of 32 rows 11.7 with 8; 4 members would prep 128 tokens
+// each, which their staging rows do not hold.)  The lines below fit these: a
+// part that is latency, and a part that grows with the rows (tokens and
+// slots) a member works on.
+int fixed_group(const ChainPlan &p, int S, int64_t n_tok) {
+  if (n_tok > kFixedMaxTok) return 0;
+  const int nblk = (S + 15) / 16;
+  // Owned slots per member: up to 64 at G = 16, up to 128 below; at most kChainTok prep tokens.
+  const auto fits = [&](int G) {
+    return (nblk + G - 1) / G * 16 <= (G == 16 ? 64 : kOwnMax) && (n_tok + G - 1) / G <= kChainTok;
+  };
+  if (p.G == 16) return fits(16) ? 16 : 0;
+  const double work = double(n_tok + S) * p.head_dim / 128;
+  const auto launches = [&](int G) { return double((p.rows + p.limit / G - 1) / (p.limit / G)); };
+  int best = 0;
+  double least = 0;
+  const auto offer = [&](int G, bool ok, double us) {
+    if (ok && (best == 0 || us < least)) {
+      best = G;
+      least = us;
+    }
+  };
+  const int rmax = p.head_dim == 128 ? RowMax<128>::value : RowMax<64>::value;
+  offer(8, fits(8), launches(8) * (5.2 + 0.0075 * work));
+  offer(4, fits(4), launches(4) * (4.0 + 0.016 * work));
+  offer(1, S <= rmax && n_tok <= rmax, launches(1) * (1.5 + 0.058 * work));
+  return best;
+}
+}  // namespace
+
 bool chain_fixed_ok(const ChainPlan &p, const ChainList &list, int64_t n_tok) {
-  if (n_tok > kFixedMaxTok || list.count < 1 || (p.G != 8 && p.G != 16)) return false;
+  if (list.count < 1) return false;
   const int S = list.state_before[0];
   for (int i = 0; i < list.count; ++i)
     if (list.n_append[i] != 0 || list.state_before[i] != S) return false;
-  // Owned slots per member: up to 64 at G = 16, up to 128 at G = 8.
-  const int nblk = (S + 15) / 16;
-  return (nblk + p.G - 1) / p.G * 16 <= (p.G == 8 ? kOwnMax : 64);
+  return fixed_group(p, S, n_tok) != 0;
 }
 
 int64_t chain_scratch_bytes(const kvm_layer &L, int64_t n_tok) {
@@ -1631,37 +2055,53 @@ hipError_t launch_chain(const kvm_layer &L, const kvm_seq &src, int64_t n_tok,
   const int rows = int(L.batch * L.kv_heads);
   const int64_t log_stride = int64_t(rows) * n_tok;
   const bool fixed = p.fixed && chain_fixed_ok(p, list, n_tok);
-  for (int row0 = 0; row0 < rows; row0 += p.row_batch) {
-    const int nrows = std::min(p.row_batch, rows - row0);
+  const int G = fixed ? fixed_group(p, list.state_before[0], n_tok) : p.G;
+  if (G == 1) {  // one independent workgroup per row
+    if (L.head_dim == 128)
+      hipLaunchKernelGGL(k_chain_row<128>, dim3(unsigned(rows)), dim3(kRowThreads), 0, stream, L, src, int(n_tok),
+                         st, snaps, list, route_log, append_log, log_stride);
+    else
+      hipLaunchKernelGGL(k_chain_row<64>, dim3(unsigned(rows)), dim3(kRowThreads), 0, stream, L, src, int(n_tok),
+                         st, snaps, list, route_log, append_log, log_stride);
+    return hipGetLastError();
+  }
+  const int row_batch = p.limit / G / 8 * 8;  // rows a launch keeps resident, one group per XCD each
+  for (int row0 = 0; row0 < rows; row0 += row_batch) {
+    const int nrows = std::min(row_batch, rows - row0);
     // Barrier counters and the abort flag start at zero in every launch.
     hipError_t e = launch_fill_u32(cs.bar, kChainMaxWorkgroups * kCounterStride + 64, 0u, stream);
     if (e != hipSuccess) return e;
-    const dim3 grid(unsigned((nrows + 7) / 8 * 8 * p.G)), blk(kChainThreads);
+    const dim3 grid(unsigned((nrows + 7) / 8 * 8 * G)), blk(kChainThreads);
     if (fixed) {
       const int nt = int(n_tok);
-      const bool own128 = ((list.state_before[0] + 15) / 16 + p.G - 1) / p.G * 16 > 64;  // G == 8 then
+      const bool own128 = ((list.state_before[0] + 15) / 16 + G - 1) / G * 16 > 64;  // G < 16 then
 #define KVM_FIXED(DD, GG, OO)                                                                               \
   hipLaunchKernelGGL((k_chain_fixed<DD, GG, OO>), grid, blk, 0, stream, L, src, nt, st, snaps, list, cs, rows, \
                      row0, nrows, route_log, append_log, log_stride)
-      if (L.head_dim == 128 && p.G == 8 && own128)
-        KVM_FIXED(128, 8, 128);
-      else if (L.head_dim == 128 && p.G == 8)
-        KVM_FIXED(128, 8, 64);
-      else if (L.head_dim == 128)
-        KVM_FIXED(128, 16, 64);
-      else if (p.G == 8 && own128)
-        KVM_FIXED(64, 8, 128);
-      else if (p.G == 8)
-        KVM_FIXED(64, 8, 64);
-      else
-        KVM_FIXED(64, 16, 64);
+#define KVM_FIXED_D(DD)            \
+  if (G == 16)                     \
+    KVM_FIXED(DD, 16, 64);         \
+  else if (G == 8 && own128)       \
+    KVM_FIXED(DD, 8, 128);         \
+  else if (G == 8)                 \
+    KVM_FIXED(DD, 8, 64);          \
+  else if (own128)                 \
+    KVM_FIXED(DD, 4, 128);         \
+  else                             \
+    KVM_FIXED(DD, 4, 64)
+      if (L.head_dim == 128) {
+        KVM_FIXED_D(128);
+      } else {
+        KVM_FIXED_D(64);
+      }
+#undef KVM_FIXED_D
 #undef KVM_FIXED
     } else if (L.head_dim == 128) {
       hipLaunchKernelGGL(k_chain<128>, grid, blk, p.dyn_lds, stream, L, src, int(n_tok), st, snaps, list, cs,
-                         rows, row0, nrows, p.G, p.tpw, p.spm_max, route_log, append_log, log_stride);
+                         rows, row0, nrows, G, p.tpw, p.spm_max, route_log, append_log, log_stride);
     } else {
       hipLaunchKernelGGL(k_chain<64>, grid, blk, p.dyn_lds, stream, L, src, int(n_tok), st, snaps, list, cs,
-                         rows, row0, nrows, p.G, p.tpw, p.spm_max, route_log, append_log, log_stride);
+                         rows, row0, nrows, G, p.tpw, p.spm_max, route_log, append_log, log_stride);
     }
     e = hipGetLastError();
     if (e != hipSuccess) return e;

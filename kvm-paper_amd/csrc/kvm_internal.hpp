@@ -117,14 +117,15 @@ struct ChainPlan {
   int G;          // workgroups per row
   int tpw;        // tokens per workgroup (multiple of 16, <= 64)
   int spm_max;    // slots per workgroup at max_slots
-  int row_batch;  // rows per launch (all rows, or batches of them when they do not fit at once)
-  int workgroups; // per launch
+  int limit;      // workgroups a launch keeps resident
+  int rows;       // rows of the call
+  int head_dim;
   size_t dyn_lds;
 };
 // False when the shape does not fit the chain (the per-update kernels then run).
 bool chain_plan(const kvm_layer &L, int64_t n_tok, int64_t max_slots, ChainPlan *p);
-// Whether a batch may use the slot-owner kernel: no appends, one state
-// length, at most 64 slots per member and 512 tokens per update.
+// Whether a batch may use the chains without appends (slot-owner or one
+// workgroup per row): no appends, one state length, and a fitting group size.
 bool chain_fixed_ok(const ChainPlan &p, const ChainList &list, int64_t n_tok);
 int64_t chain_scratch_bytes(const kvm_layer &L, int64_t n_tok);
 ChainScratch carve_chain_scratch(void *base, const kvm_layer &L, int64_t n_tok);

@@ -1004,3 +1004,39 @@ def test_prefill_saturation_budget_matches_oracle(lib):
         total += g_sel.numel()
     T.log(f"[prefill-saturation] S {C} -> {S}, {len(rec.updates)} updates, {n_diff}/{total} merge routes differ")
     assert n_diff == 0
+
+
+@pytest.mark.parametrize("B,Hkv,Tn,D,C,skew", [
+    (5, 8, 2100, 128, 256, False),   # 40 rows: four members per row
+    (5, 8, 2100, 128, 256, True),
+    (8, 9, 1000, 64, 128, False),    # 72 rows of 64-wide heads
+    (9, 33, 1500, 128, 256, False),  # 297 rows: one workgroup per row, more rows than compute units
+    (9, 33, 1500, 128, 256, True),
+    (16, 16, 700, 128, 100, False),  # one workgroup per row, ragged chunk
+    (16, 16, 330, 64, 17, False),    # a single token tile and slot block, mostly empty
+    (16, 16, 2600, 64, 512, True),   # the largest slots and chunk of 64-wide heads
+])
+def test_chain_many_rows_matches_per_update_kernels(lib, monkeypatch, B, Hkv, Tn, D, C, skew):
+    """Chains without appends over more rows than eight members per row keep
+    resident (four members per row, or one workgroup per row): routes, state
+    and outputs must equal the per-update kernels bit for bit."""
+    T.log(f"[chain-rows] B{B} Hkv{Hkv} T{Tn} D{D} C{C} skew {skew}")
+    cfg = T.mixer_config(Hkv, Hkv, D, C, mode="fixed", sink=1, min_len=C, n_max=4, factor=6.0)
+    gen = torch.Generator().manual_seed(3)
+    ln_w = (1 + 0.1 * torch.randn(D, generator=gen)).bfloat16()
+    ln_b = (0.1 * torch.randn(D, generator=gen)).bfloat16()
+    m = T.make_mixer(cfg, ln_w, ln_b, torch.ones(Hkv), torch.ones(Hkv))
+    q, k, v, g = _random_inputs(B, Hkv, Hkv, Tn, D, 31)
+    if skew:
+        d = torch.randn(D, generator=gen)
+        k = (d / d.norm() + 0.02 * torch.randn(B, Hkv, Tn, D, generator=gen) / math.sqrt(D)).bfloat16()
+    q, k, v, g = (t.to(DEV) for t in (q, k, v, g))
+    res = {}
+    for chain in ("1", "0"):
+        monkeypatch.setenv("KVM_AMD_CHAIN", chain)
+        with torch.no_grad():
+            res[chain] = m.prefill_raw(q, k, v, g, route_log=True)
+        torch.cuda.synchronize()
+    assert res["1"]["plan"].n_updates > 0
+    for key in ("route_log", "append_log", "out", "state_k", "state_v", "state_vlen", "state_k_attn", "state_v_attn"):
+        assert torch.equal(res["1"][key], res["0"][key]), key
