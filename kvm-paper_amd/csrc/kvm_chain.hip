@@ -31,18 +31,24 @@
 // compute units for longer than the poll budget makes the waits time out;
 // the result is then reported, never silently used.
 //
-// Work split of one update of a row:
-//   member m owns tokens [m * tpw, (m + 1) * tpw)  (prep, novelty, append,
-//                routing; tpw <= 64, the token operands stay in LDS)
-//   member m owns slots  [m * spm, (m + 1) * spm)  (merge sums, refreshed
-//                attention rows), spm = ceil(slots / G)
+// Work split of one update of a row in k_chain (batches with appends):
+//   member m owns tokens [m * tpw, (m + 1) * tpw)  (prep, append; tpw <= 64)
+//   member m owns the 16-slot blocks m, m + G, ... (their attention keys in
+//                LDS; scores of every token, merge sums, refreshed rows)
 // Phases, separated by group barriers (|):
-//   [novelty -> | -> rank, append my tokens -> |] -> route(my tokens) -> |
-//   -> merge(my slots) -> arrive, prep(my tokens of the next update), wait
-// The raw keys / values of the next update's tokens are loaded while the
-// routing scan runs, and the merge keys / values alternate between two
-// buffers, so the next update's prep overlaps the barrier that ends this
-// update.
+//   [novelty over my slots -> | -> select, append my tokens -> |]
+//   -> route over my slots, prep(my tokens of the next update) -> |
+//   -> combine, lists, merge(my slots)
+// Every member scores every token against its own slots only, so an update
+// reads each slot row once, from LDS (a split by tokens had every member read
+// every slot row from L2 for its 32 tokens, twice), and the members exchange
+// one maximum per token and scan.  The next update's rows are stored before a
+// member publishes its routes, so no barrier ends an update.
+// Bound by latency (barriers, L2 round trips) and, at thousands of slots, by
+// the merge's row traffic.  us per update: 32 rows, C 256, 256 to 2015 slots,
+// 51 -> 31.5 (novelty 7, selection 1.7, route 3, lists 2.5, merge 7, three
+// barriers 2 each); 16 rows of 64-wide heads, C 128, up to 849 slots, 23.3 ->
+// 17.7; 8 rows, up to 1024 slots, 23.5 -> 17.4.
 // The state (s_k, s_v, s_vlen) lives in the caller's arrays; snapshot u
 // holds the attention rows routing reads and snapshot u + 1 receives the
 // refreshed rows of every slot, as in the per-update path.
@@ -52,6 +58,7 @@
 #include "kvm_seq.hpp"
 
 #include <algorithm>
+#include <type_traits>
 
 namespace kvm {
 
@@ -81,6 +88,19 @@ __device__ unsigned long long g_chain_ts[2][128][16];
 
 namespace {
 
+// Dynamic LDS of the appending chain: the scans' maxima, or the lists' counts in their place ...
+__host__ __device__ inline int append_red_bytes(int n_tok, int own_cap) {
+  int ntg = 64;
+  while (ntg < n_tok) ntg <<= 1;
+  const int scan = (ntg < 512 ? 512 : ntg) * 8, lists = (n_tok + 63) / 64 * own_cap * 2;
+  return ((scan > lists ? scan : lists) + 15) & ~15;
+}
+// ... then off / cnt [own_cap] and sorted / apos [n_tok].
+__host__ __device__ inline int append_lds_bytes(int n_tok, int own_cap) {
+  return append_red_bytes(n_tok, own_cap) + 4 * own_cap + 4 * n_tok;
+}
+
+constexpr int kAppendDynLds = 44 * 1024;  // beside the attention keys (OwnLds)
 constexpr int kChainThreads = 512;
 constexpr int kChainWaves = kChainThreads / 64;
 constexpr int kChainTok = 64;        // tokens per member at most
@@ -230,137 +250,6 @@ __device__ __forceinline__ AttnRows snap_at(const SnapRing &r, int64_t idx) {
   return AttnRows{r.k + o, r.v + o, r.cap};
 }
 
-// Scan of the member's tokens (operand rows in LDS, ntk <= 64 of them)
-// against slots [0, hi) of one row's attention keys (written by other
-// members) on MFMA 16x16x32 bf16, computed transposed (slot x token) with
-// the same operand roles and k-step order as the per-update routing kernel,
-// so the fp32 scores are bit-identical.  Wave w takes the 16-slot tiles
-// w + 8 * (4p + s), s < 4, in pass p and loads a pass's four tiles at once;
-// `hook` runs once, right after the first pass's loads are issued.
-//   NOVELTY: max over slots of the bf16-rounded score
-//            (model/kvm_mixer.py:66-68);
-//   route:   first argmax of the fp32 score over slots [lo, hi)
-//            (model/kvm_fp32_routing_reference.py:30-34).
-// Result of local token lt: best_v[lt] (and best_i[lt]).
-template <int D, bool NOVELTY, typename Hook>
-__device__ __forceinline__ void scan_slots(const uint16_t *op, const uint16_t *keys, int lo,
-                                           int hi, int ntk, float (*red_v)[kChainTok],
-                                           int (*red_i)[kChainTok], float *best_v, int *best_i,
-                                           Hook &&hook) {
-  constexpr int STR = D + 8;
-  constexpr int KS = D / 32;
-  constexpr int TF = kTilesInFlight;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int n_tt = (ntk + 15) >> 4;
-  const int n_st = (hi + 15) >> 4;
-  // Rows j >= hi lie past the resource and read zero (and are masked).
-  const __amdgpu_buffer_rsrc_t kr = l2_rsrc(keys, int64_t(hi) * D * 2);
-
-  float best[4];
-  int bidx[4];
-#pragma unroll
-  for (int tt = 0; tt < 4; ++tt) {
-    best[tt] = -INFINITY;
-    bidx[tt] = -1;
-  }
-  for (int p0 = 0; p0 < n_st; p0 += kChainWaves * TF) {
-    uint4 a[TF][KS];
-#pragma unroll
-    for (int s = 0; s < TF; ++s) {
-      const int j = (p0 + wave + kChainWaves * s) * 16 + (lane & 15);
-#pragma unroll
-      for (int ks = 0; ks < KS; ++ks) a[s][ks] = l2_ld16(kr, (j * D + ks * 32 + (lane >> 4) * 8) * 2);
-    }
-    if (p0 == 0) hook();
-#pragma unroll
-    for (int tt = 0; tt < 4; ++tt) {
-      if (tt < n_tt) {
-        bf16x8 bx[KS];
-#pragma unroll
-        for (int ks = 0; ks < KS; ++ks)
-          bx[ks] = as_bf16x8(*reinterpret_cast<const uint4 *>(
-              &op[(tt * 16 + (lane & 15)) * STR + ks * 32 + (lane >> 4) * 8]));
-        f32x4 acc[TF];
-#pragma unroll
-        for (int s = 0; s < TF; ++s) acc[s] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int ks = 0; ks < KS; ++ks)
-#pragma unroll
-          for (int s = 0; s < TF; ++s)
-            acc[s] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(a[s][ks]), bx[ks], acc[s], 0,
-                                                             0, 0);
-        // Slots in increasing order within the lane: a strict > keeps the
-        // first maximum.
-#pragma unroll
-        for (int s = 0; s < TF; ++s) {
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            const int j = (p0 + wave + kChainWaves * s) * 16 + (lane >> 4) * 4 + i;
-            // Selects, not branches: slots outside [lo, hi) score -inf.
-            if constexpr (NOVELTY) {
-              best[tt] = fmaxf(best[tt], j < hi ? rbf(acc[s][i]) : -INFINITY);
-            } else {
-              const float sc = (j >= lo) & (j < hi) ? acc[s][i] : -INFINITY;
-              const bool take = sc > best[tt];
-              best[tt] = take ? sc : best[tt];
-              bidx[tt] = take ? j : bidx[tt];
-            }
-          }
-        }
-      }
-    }
-  }
-  if (n_st == 0) hook();
-
-  // Lane groups (slots 4q..4q+3 of every tile), then waves (interleaved
-  // tiles): larger score wins, equal scores go to the lower slot.
-#pragma unroll
-  for (int tt = 0; tt < 4; ++tt) {
-    float bv = best[tt];
-    int bi = bidx[tt];
-#pragma unroll
-    for (int r = 0; r < 2; ++r) {
-      const uint32_t vb = __float_as_uint(bv), ib = uint32_t(bi);
-      const float ob = __uint_as_float(r == 0 ? xor16_lane(vb, lane) : xor32_lane(vb, lane));
-      const int oi = int(r == 0 ? xor16_lane(ib, lane) : xor32_lane(ib, lane));
-      if constexpr (NOVELTY) {
-        bv = fmaxf(bv, ob);
-      } else if (oi >= 0 && (bi < 0 || ob > bv || (ob == bv && oi < bi))) {
-        bv = ob;
-        bi = oi;
-      }
-    }
-    if (lane < 16) {
-      red_v[wave][tt * 16 + lane] = bv;
-      red_i[wave][tt * 16 + lane] = bi;
-    }
-  }
-  __syncthreads();
-  if (tid < kChainTok) {
-    float vv[kChainWaves];
-    int ii[kChainWaves];
-#pragma unroll
-    for (int w = 0; w < kChainWaves; ++w) {
-      vv[w] = red_v[w][tid];
-      ii[w] = red_i[w][tid];
-    }
-    float bv = vv[0];
-    int bi = ii[0];
-#pragma unroll
-    for (int w = 1; w < kChainWaves; ++w) {
-      if constexpr (NOVELTY) {
-        bv = fmaxf(bv, vv[w]);
-      } else if (ii[w] >= 0 && (bi < 0 || vv[w] > bv || (vv[w] == bv && ii[w] < bi))) {
-        bv = vv[w];
-        bi = ii[w];
-      }
-    }
-    best_v[tid] = bv;
-    if (best_i) best_i[tid] = bi;
-  }
-  __syncthreads();
-}
-
 // Raw key / value / gate of the member's tokens, D/8 lanes per token.
 template <int D>
 struct RawTok {
@@ -369,38 +258,45 @@ struct RawTok {
   uint16_t g[IT];  // bf16 bits, converted where used (no wait at the load)
 };
 
+// Slot of a member's local slot l: the member owns 16-slot blocks m, m + G, ...
+__device__ __forceinline__ int own_local_to_slot(int l, int G, int m) {
+  return (((l >> 4) * G + m) << 4) | (l & 15);
+}
+
+// Own slots whose attention keys the appending chain keeps in LDS; further
+// ones are read from their snapshot.
 template <int D>
+struct OwnLds {
+  static constexpr int value = D == 128 ? 384 : 768;
+};
+
+template <int D, int G>
 __global__ __launch_bounds__(kChainThreads) void k_chain(
     kvm_layer L, kvm_seq src, int n_tok, kvm_state st, SnapRing snaps, ChainList list,
-    ChainScratch cs, int rows, int row0, int nrows, int G, int tpw, int spm_max, int32_t *route_log,
+    ChainScratch cs, int rows, int row0, int nrows, int tpw, int own_cap, int32_t *route_log,
     int32_t *append_log, int64_t log_stride) {
   constexpr int GL = D / 8;                 // lanes per D-wide row
   constexpr int STR = D + 8;                // LDS row stride (elements)
+  constexpr int KS = D / 32;
   constexpr int RPP = kChainThreads / GL;   // rows per pass
   constexpr int IT = RawTok<D>::IT;         // passes over the member's tokens
+  constexpr int OWNL = OwnLds<D>::value;
   static_assert(IT * RPP == kChainTok, "token passes");
-  __shared__ __attribute__((aligned(16))) uint16_t op_r[kChainTok * STR];  // merge keys
-  __shared__ __attribute__((aligned(16))) uint16_t op_n[kChainTok * STR];  // prep(k)
-  __shared__ float red_v[kChainWaves][kChainTok];
-  __shared__ int red_i[kChainWaves][kChainTok];
-  __shared__ float res_v[kChainTok];
-  __shared__ int res_i[kChainTok];
+  __shared__ __attribute__((aligned(16))) uint16_t own_k[OWNL * STR];  // attention keys of my slots
+  __shared__ int wtot[kChainWaves];
   __shared__ int ok_lds;
   __shared__ float ln_w[D], ln_b[D];  // ln_s_k parameters (LDS: no wait on global loads)
-  extern __shared__ __attribute__((aligned(16))) int dyn[];
-  int *tok_a = dyn;               // [n_tok] novelty rank flag
-  int *mr = tok_a + n_tok;        // [n_tok] local slot of each token or -1
-  int *lst = mr + n_tok;          // [n_tok] tokens placed per slot
-  int *sorted = lst + n_tok;      // [n_tok] per-slot lists in token order
-  int *cnt = sorted + n_tok;      // [spm_max]
-  int *off = cnt + spm_max;       // [spm_max]
-  int *fill = off + spm_max;      // [spm_max]
-  int *apos = sorted;             // [n_tok] append position of each token (append phase)
-  // [npow] sort keys of the append selection, 8-byte aligned after fill
-  const int npow = n_tok <= 1 ? 1 : 1 << (32 - __builtin_clz(unsigned(n_tok - 1)));
-  uint64_t *skey = reinterpret_cast<uint64_t *>(fill + spm_max + (spm_max & 1));
+  // [slot group][token] maxima of a scan (8 bytes each); in their place, the
+  // lists' counts [64 tokens][own_cap].  Then off / cnt [own_cap], sorted and
+  // apos [n_tok] (append_lds_bytes).
+  extern __shared__ __attribute__((aligned(16))) uint64_t red[];
+  uint16_t *const wsc = reinterpret_cast<uint16_t *>(red);
+  uint16_t *const off = wsc + append_red_bytes(n_tok, own_cap) / 2, *const cnt = off + own_cap;
+  uint16_t *const sorted = cnt + own_cap;                              // tokens of my slots, slot by slot
+  int16_t *const apos = reinterpret_cast<int16_t *>(sorted + n_tok);   // append position of a token or -1
 
-  const int tid = threadIdx.x, part = tid % GL;
+  const int tid = threadIdx.x, lane = tid & 63, part = tid % GL, sub = tid / GL;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int xcd = blockIdx.x & 7, q = blockIdx.x >> 3;
   const int member = q % G, group = (q / G) * 8 + xcd;
   if (group >= nrows) return;
@@ -408,13 +304,13 @@ __global__ __launch_bounds__(kChainThreads) void k_chain(
     ln_w[d] = static_cast<const float *>(L.ln_weight)[d];
     ln_b[d] = static_cast<const float *>(L.ln_bias)[d];
   }
-  __syncthreads();
   const int row = row0 + group;  // this launch serves rows row0 .. row0 + nrows - 1
   const int b = row / int(L.kv_heads), h = row % int(L.kv_heads);
   const int t0 = member * tpw;
   const int ntk = max(0, min(n_tok, t0 + tpw) - t0);
   const int64_t rb = int64_t(row) * n_tok;
-  const int64_t par_stride = int64_t(rows) * n_tok * D;  // elements between the two merge buffers
+  const int64_t buf_stride = int64_t(rows) * n_tok * D;  // elements between merge buffers
+  const int rowb = n_tok * D * 2;                        // bytes of a row's tokens in one of them
   unsigned *ctr = cs.bar + group * kCounterStride;
   unsigned target = 0;
   auto arrive = [&]() __attribute__((always_inline)) {
@@ -428,6 +324,13 @@ __global__ __launch_bounds__(kChainThreads) void k_chain(
   uint16_t *s_v = static_cast<uint16_t *>(st.s_v);
   float *s_vlen = static_cast<float *>(st.s_vlen);
   const int64_t srow = int64_t(row) * st.capacity;
+  // Token rows of update i: merge keys and values in buffers 0..2 of gk / gv
+  // (an update's are prepared one update ahead and read last by its merge,
+  // while the next but one may already be prepared by another member);
+  // prep(k) of appending updates in buffer 3 of gk (even) or gv (odd).
+  auto gk_of = [&](int i) __attribute__((always_inline)) { return cs.gk + (i % 3) * buf_stride + rb * D; };
+  auto gv_of = [&](int i) __attribute__((always_inline)) { return cs.gv + (i % 3) * buf_stride + rb * D; };
+  auto pk_of = [&](int i) __attribute__((always_inline)) { return ((i & 1) ? cs.gv : cs.gk) + 3 * buf_stride + rb * D; };
 
   // Raw tokens of update i (token 0 of the chunk for idle lanes).  Prefill
   // tokens never come from a ring (src.ring == 0, checked by the host).
@@ -438,7 +341,8 @@ __global__ __launch_bounds__(kChainThreads) void k_chain(
     const int64_t tb = list.tok_begin[i];
 #pragma unroll
     for (int it = 0; it < IT; ++it) {
-      const int lt = (tid + it * kChainThreads) / GL;
+      if (it * RPP >= ntk) break;  // uniform
+      const int lt = it * RPP + sub;
       const int64_t t = tb + (lt < ntk ? t0 + lt : 0);
       rt.k[it] = ld_stream16(k_row + t * src.k_st + part * 8);
       rt.v[it] = ld_stream16(v_row + t * src.v_st + part * 8);
@@ -446,16 +350,14 @@ __global__ __launch_bounds__(kChainThreads) void k_chain(
     }
   };
   // prep (model/kvm_mixer.py:120-129, model/kvm_triton_mixer.py:429-446):
-  // merge key / value of my tokens into LDS (routing operand) and into the
-  // update's merge buffer; prep(k) into LDS when the update appends.
+  // merge key / value rows of my tokens, and prep(k) when the update appends.
   auto prep = [&](int i, const RawTok<D> &rt) __attribute__((always_inline)) {
     const bool nov = list.n_append[i] > 0;
-    uint16_t *gkb = cs.gk + (i & 1) * par_stride;
-    uint16_t *gvb = cs.gv + (i & 1) * par_stride;
+    uint16_t *gkb = gk_of(i), *gvb = gv_of(i), *pkb = pk_of(i);
 #pragma unroll
     for (int it = 0; it < IT; ++it) {
-      const int lt = (tid + it * kChainThreads) / GL;
-      const bool valid = lt < ntk;
+      if (it * RPP >= ntk) break;  // uniform
+      const int lt = it * RPP + sub;
       float k[8], v[8];
       unpack8(rt.k[it], k);
       unpack8(rt.v[it], v);
@@ -467,21 +369,145 @@ __global__ __launch_bounds__(kChainThreads) void k_chain(
         gk[e] = L.gate_keys ? rbf(k[e] * g) : k[e];
         gv[e] = L.gate_values ? rbf(v[e] * g) : v[e];
       }
-      const uint4 z = make_uint4(0, 0, 0, 0);
-      *reinterpret_cast<uint4 *>(&op_r[lt * STR + part * 8]) = valid ? pack8(gk) : z;
-      if (nov) *reinterpret_cast<uint4 *>(&op_n[lt * STR + part * 8]) = valid ? pack8(k) : z;
-      if (valid) {
-        const int64_t o = (rb + t0 + lt) * D + part * 8;
+      if (lt < ntk) {
+        const int64_t o = int64_t(t0 + lt) * D + part * 8;
         store8(gkb + o, gk);
         store8(gvb + o, gv);
+        if (nov) store8(pkb + o, k);
+      }
+    }
+  };
+
+  // ---- attention keys of my slots (those of the first OWNL) into LDS.
+  auto load_own = [&](const uint16_t *keys, int lo, int hi) __attribute__((always_inline)) {
+    const __amdgpu_buffer_rsrc_t kr = l2_rsrc(keys, int64_t(hi) * D * 2);
+    for (int l = sub; l < min(own_cap, OWNL); l += RPP) {
+      const int j = own_local_to_slot(l, G, member);
+      if (j >= lo && j < hi)
+        *reinterpret_cast<uint4 *>(&own_k[l * STR + part * 8]) = l2_ld16(kr, (j * D + part * 8) * 2);
+    }
+  };
+  {
+    const AttnRows a0 = snap_at(snaps, list.u0);
+    load_own(a0.k + int64_t(row) * a0.cap * D, 0, list.state_before[0]);
+  }
+  // The scans' work split: token groups of 64 (waves tg, tg + 8, ...) x slot
+  // groups (interleaved blocks of 16) over the waves.
+  int ntg = 1;
+  while (ntg * 64 < n_tok) ntg <<= 1;
+  const int nsg = max(1, kChainWaves / ntg), sg = wave / ntg, tg0 = wave % ntg;
+
+  // Scan of every token (rows at `tok`, prepared by all members) against my
+  // slots below hi on MFMA 16x16x32 bf16, computed transposed (slot x token)
+  // with the same operand roles and k-step order as the per-update routing
+  // kernel, so the fp32 scores are bit-identical.  Into red[slot group][token]:
+  //   NOVELTY: maximum of the bf16-rounded score, as float bits
+  //            (model/kvm_mixer.py:66-68);
+  //   route:   route key of the first argmax over slots [lo, hi)
+  //            (model/kvm_fp32_routing_reference.py:30-34).
+  // The caller has loaded bx for the wave's first token group.
+  uint4 bx[4][KS];
+  auto load_bx = [&](const uint16_t *tok, int tg) __attribute__((always_inline)) {
+    const __amdgpu_buffer_rsrc_t tr = l2_rsrc(tok, rowb);
+#pragma unroll
+    for (int tt = 0; tt < 4; ++tt)
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks)
+        bx[tt][ks] = l2_ld16(tr, ((tg * 64 + tt * 16 + (lane & 15)) * D + ks * 32 + (lane >> 4) * 8) * 2);
+  };
+  auto scan = [&](auto novelty, const uint16_t *tok, const uint16_t *keys, int lo,
+                  int hi) __attribute__((always_inline)) {
+    constexpr bool NOVELTY = decltype(novelty)::value;
+    const __amdgpu_buffer_rsrc_t kr = l2_rsrc(keys, int64_t(hi) * D * 2);
+    const int nblk = (hi + 15) >> 4;
+    for (int tg = tg0; tg * 64 < n_tok; tg += kChainWaves) {
+      if (tg != tg0) load_bx(tok, tg);
+      float best[4];
+      int bidx[4];
+#pragma unroll
+      for (int tt = 0; tt < 4; ++tt) {
+        best[tt] = -INFINITY;
+        bidx[tt] = -1;
+      }
+      for (int lb = sg; lb * G + member < nblk; lb += nsg) {
+        const int jb = (lb * G + member) * 16;  // first slot of the block
+        uint4 a[KS];
+        if (lb * 16 < OWNL) {  // uniform
+#pragma unroll
+          for (int ks = 0; ks < KS; ++ks)
+            a[ks] = *reinterpret_cast<const uint4 *>(
+                &own_k[(lb * 16 + (lane & 15)) * STR + ks * 32 + (lane >> 4) * 8]);
+        } else {
+#pragma unroll
+          for (int ks = 0; ks < KS; ++ks)
+            a[ks] = l2_ld16(kr, ((jb + (lane & 15)) * D + ks * 32 + (lane >> 4) * 8) * 2);
+        }
+        f32x4 accs[4];
+#pragma unroll
+        for (int tt = 0; tt < 4; ++tt) accs[tt] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+          for (int tt = 0; tt < 4; ++tt)
+            accs[tt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(a[ks]), as_bf16x8(bx[tt][ks]), accs[tt], 0,
+                                                               0, 0);
+        const int j0 = jb + (lane >> 4) * 4;
+        if (jb < lo || jb + 16 > hi) {  // slots outside [lo, hi) never count
+#pragma unroll
+          for (int tt = 0; tt < 4; ++tt)
+#pragma unroll
+            for (int x = 0; x < 4; ++x)
+              accs[tt][x] = (j0 + x >= lo) & (j0 + x < hi) ? accs[tt][x] : -INFINITY;
+        }
+#pragma unroll
+        for (int tt = 0; tt < 4; ++tt) {
+          const f32x4 acc = accs[tt];
+          if constexpr (NOVELTY) {
+            // The rounding is monotone, so the maximum may be taken first.
+            best[tt] = fmaxf(best[tt], fmaxf(fmaxf(acc[0], acc[1]), fmaxf(acc[2], acc[3])));
+          } else {
+            // The lane's four slots as a tree (the earlier keeps ties), then
+            // against the running maximum: the first maximum in slot order.
+            const bool t1 = acc[1] > acc[0], t3 = acc[3] > acc[2];
+            const float v01 = t1 ? acc[1] : acc[0], v23 = t3 ? acc[3] : acc[2];
+            const int i01 = t1 ? 1 : 0, i23 = t3 ? 3 : 2;
+            const bool th = v23 > v01;
+            const float vh = th ? v23 : v01;
+            const bool take = vh > best[tt];
+            best[tt] = take ? vh : best[tt];
+            bidx[tt] = take ? j0 + (th ? i23 : i01) : bidx[tt];
+          }
+        }
+      }
+#pragma unroll
+      for (int tt = 0; tt < 4; ++tt) {
+        uint64_t *const out = &red[(sg * ntg + tg) * 64 + tt * 16 + (lane & 15)];
+        if constexpr (NOVELTY) {
+          float v = best[tt];
+          v = fmaxf(v, __uint_as_float(xor16_lane(__float_as_uint(v), lane)));
+          v = fmaxf(v, __uint_as_float(xor32_lane(__float_as_uint(v), lane)));
+          if (lane < 16) *out = __float_as_uint(rbf(v));
+        } else {
+          uint64_t key = bidx[tt] >= 0 ? route_key(best[tt], bidx[tt]) : 0;
+#pragma unroll
+          for (int r = 0; r < 2; ++r) {
+            const uint32_t hi32 = uint32_t(key >> 32), lo32 = uint32_t(key);
+            const uint64_t other = r == 0 ? (uint64_t(xor16_lane(hi32, lane)) << 32) | xor16_lane(lo32, lane)
+                                          : (uint64_t(xor32_lane(hi32, lane)) << 32) | xor32_lane(lo32, lane);
+            key = other > key ? other : key;
+          }
+          if (lane < 16) *out = key;
+        }
       }
     }
   };
 
   RawTok<D> rt;
   load_raw(0, rt);
-  prep(0, rt);
   __syncthreads();
+  prep(0, rt);
+  arrive();
+  if (!wait()) return;
 
   for (int i = 0; i < list.count; ++i) {
     const int64_t u = int64_t(list.u0) + i;
@@ -489,324 +515,351 @@ __global__ __launch_bounds__(kChainThreads) void k_chain(
     const int sb = list.state_before[i], na = list.n_append[i];
     const int s_after = sb + na;
     const int protect = min(int(L.sink_len), s_after);
+    const bool more = i + 1 < list.count;
     const AttnRows cur = snap_at(snaps, u), nxt = snap_at(snaps, u + 1);
-    const uint16_t *gkb = cs.gk + (i & 1) * par_stride;
-    const uint16_t *gvb = cs.gv + (i & 1) * par_stride;
     int32_t *rlog = route_log ? route_log + u * log_stride + rb : nullptr;
     int32_t *alog = append_log ? append_log + u * log_stride + rb : nullptr;
-    const uint16_t *cur_k = cur.k + int64_t(row) * cur.cap * D;
+    uint16_t *cur_k = cur.k + int64_t(row) * cur.cap * D, *cur_v = cur.v + int64_t(row) * cur.cap * D;
     KVM_TS_A(0);
 
     // ---- append (model/kvm_mixer.py:44-75, 231-248): the n_append least
     // novel tokens, ties to the lower index, become slots sb.. in token order.
     if (na > 0) {
-      scan_slots<D, true>(op_n, cur_k, 0, sb, ntk, red_v, red_i, res_v, nullptr, [] {});
-      if (tid < ntk) cs.nov[rb + t0 + tid] = res_v[tid];
+      load_bx(pk_of(i), tg0);
+      scan(std::true_type{}, pk_of(i), cur_k, 0, sb);
+      load_bx(gk_of(i), tg0);  // the route's operands, in flight through the append
+      __syncthreads();
+      for (int t = tid; t < n_tok; t += kChainThreads) {
+        float v = -INFINITY;
+        for (int x = 0; x < nsg; ++x) v = fmaxf(v, __uint_as_float(uint32_t(red[x * ntg * 64 + t])));
+        cs.nov[(rb + t) * G + member] = v;
+      }
       KVM_TS_A(1);
       arrive();
       if (!wait()) return;
       KVM_TS_A(2);
-      // The na smallest (novelty, token) pairs: a bitonic sort of the unique
-      // keys mono(novelty) << 32 | token (the same order as comparing the
-      // novelty, then the index; -0 is read as +0 so that it ties with it),
-      // padded with the largest key to a power of two.
-      const __amdgpu_buffer_rsrc_t nr = l2_rsrc(cs.nov + rb, int64_t(n_tok) * 4);
-      for (int t = tid; t < npow; t += kChainThreads) {
-        uint64_t key = ~uint64_t(0);
-        if (t < n_tok) {
-          const float x = __uint_as_float(l2_ld4(nr, t * 4)) + 0.0f;
-          const uint32_t bits = __float_as_uint(x);
-          const uint32_t m = (bits & 0x80000000u) ? ~bits : (bits | 0x80000000u);
-          key = (uint64_t(m) << 32) | uint32_t(t);
+      // The na tokens of smallest (novelty, token), on wave 0: the novelties
+      // are bf16 values, so their order is that of 16-bit keys (-0 read as
+      // +0); the largest key to take is found bit by bit with ballots, and
+      // among its tokens the first ones in token order are taken.
+      uint32_t *const nkey = reinterpret_cast<uint32_t *>(red);  // [16 * 64]: the maxima have been published
+      {
+        const __amdgpu_buffer_rsrc_t nr = l2_rsrc(cs.nov + rb * G, int64_t(n_tok) * G * 4);
+        for (int t = tid; t < ntg * 64; t += kChainThreads) {
+          uint4 p4[G / 4];  // past the tokens: zeros, not used
+#pragma unroll
+          for (int m = 0; m < G / 4; ++m) p4[m] = l2_ld16(nr, (t * G + m * 4) * 4);
+          float v = -INFINITY;
+#pragma unroll
+          for (int m = 0; m < G / 4; ++m)
+            v = fmaxf(v, fmaxf(fmaxf(__uint_as_float(p4[m].x), __uint_as_float(p4[m].y)),
+                               fmaxf(__uint_as_float(p4[m].z), __uint_as_float(p4[m].w))));
+          const uint32_t bits = __float_as_uint(v + 0.0f);
+          const uint32_t key = ((bits & 0x80000000u) ? ~bits : (bits | 0x80000000u)) >> 16;
+          nkey[t] = t < n_tok ? key : 0xffffffffu;  // above every novelty
         }
-        skey[t] = key;
-        if (t < n_tok) tok_a[t] = 0;
       }
       __syncthreads();
-      // Keys tid and tid + 512 in registers: a compare-exchange stage whose
-      // partner distance j is below 64 pairs keys of one wave (e ^ j is in
-      // e's 64-key block) and runs on lane shuffles; the others go through
-      // LDS, a barrier each.
-      constexpr int KPT = 2;  // keys per thread (n_tok <= 1024)
-      uint64_t rk[KPT];
-      auto load_keys = [&]() __attribute__((always_inline)) {
+      if (wave == 0) {
+        auto select = [&](auto groups) __attribute__((always_inline)) {
+          constexpr int NV = decltype(groups)::value;  // tokens per lane
+          uint32_t key[NV];
 #pragma unroll
-        for (int x = 0; x < KPT; ++x) {
-          const int e = tid + x * kChainThreads;
-          rk[x] = e < npow ? skey[e] : ~uint64_t(0);
-        }
-      };
-      auto store_keys = [&]() __attribute__((always_inline)) {
+          for (int x = 0; x < NV; ++x) key[x] = nkey[x * 64 + lane];
+          uint32_t cut = 0;
+          int left = na;  // tokens to take among those that agree with cut so far
 #pragma unroll
-        for (int x = 0; x < KPT; ++x) {
-          const int e = tid + x * kChainThreads;
-          if (e < npow) skey[e] = rk[x];
-        }
-      };
-      load_keys();
-      for (int k2 = 2; k2 <= npow; k2 <<= 1) {
-        int j = k2 >> 1;
-        if (j >= 64) {
-          store_keys();
-          __syncthreads();
-          for (; j >= 64; j >>= 1) {
-            for (int e = tid; e < npow; e += kChainThreads) {
-              const int f = e ^ j;
-              if (f > e) {
-                const uint64_t a = skey[e], c = skey[f];
-                if ((a > c) == ((e & k2) == 0)) {
-                  skey[e] = c;
-                  skey[f] = a;
-                }
-              }
+          for (int bit = 15; bit >= 0; --bit) {
+            int n = 0;
+#pragma unroll
+            for (int x = 0; x < NV; ++x) n += __popcll(__ballot((key[x] >> bit) == (cut >> bit)));
+            if (n < left) {
+              left -= n;
+              cut |= 1u << bit;
             }
-            __syncthreads();
           }
-          load_keys();
-        }
-        for (; j > 0; j >>= 1) {
+          int base = 0;
 #pragma unroll
-          for (int x = 0; x < KPT; ++x) {
-            const int e = tid + x * kChainThreads;
-            const uint32_t lo = uint32_t(__shfl_xor(int(uint32_t(rk[x])), j));
-            const uint32_t hi = uint32_t(__shfl_xor(int(uint32_t(rk[x] >> 32)), j));
-            const uint64_t o = (uint64_t(hi) << 32) | lo;
-            // The lower index of an ascending pair keeps the smaller key.
-            const bool take_min = ((e & k2) == 0) == ((e & j) == 0);
-            const uint64_t mn = rk[x] < o ? rk[x] : o, mx = rk[x] < o ? o : rk[x];
-            if (e < npow) rk[x] = take_min ? mn : mx;
+          for (int x = 0; x < NV; ++x) {
+            const uint64_t tie = __ballot(key[x] == cut);
+            const int before = int(__builtin_amdgcn_mbcnt_hi(
+                uint32_t(tie >> 32), __builtin_amdgcn_mbcnt_lo(uint32_t(tie), 0u)));
+            const bool ap = key[x] < cut || (key[x] == cut && before < left);
+            left -= min(left, int(__popcll(tie)));
+            const uint64_t bal = __ballot(ap);
+            const int at = base + int(__builtin_amdgcn_mbcnt_hi(
+                                      uint32_t(bal >> 32), __builtin_amdgcn_mbcnt_lo(uint32_t(bal), 0u)));
+            base += int(__popcll(bal));
+            if (x * 64 + lane < n_tok) apos[x * 64 + lane] = int16_t(ap ? at : -1);
           }
-        }
+        };
+        if (ntg == 1)
+          select(std::integral_constant<int, 1>{});
+        else if (ntg == 2)
+          select(std::integral_constant<int, 2>{});
+        else if (ntg == 4)
+          select(std::integral_constant<int, 4>{});
+        else if (ntg == 8)
+          select(std::integral_constant<int, 8>{});
+        else
+          select(std::integral_constant<int, 16>{});
       }
-      store_keys();
-      __syncthreads();
-      for (int r = tid; r < na; r += kChainThreads) tok_a[int(uint32_t(skey[r]))] = 1;
       __syncthreads();
       KVM_TS_A(3);
-      // Append position of every appended token: the appended tokens before
-      // it, by wave ballots in token order (wave totals in res_v).
-      {
-        int base = 0;
-        for (int c0 = 0; c0 < n_tok; c0 += kChainThreads) {
-          const int t = c0 + tid;
-          const bool ap = t < n_tok && tok_a[t] != 0;
-          const uint64_t bal = __ballot(ap);
-          const int before = int(__builtin_amdgcn_mbcnt_hi(uint32_t(bal >> 32),
-                                                           __builtin_amdgcn_mbcnt_lo(uint32_t(bal), 0u)));
-          if ((tid & 63) == 0) res_v[tid >> 6] = __int_as_float(__popcll(bal));
-          __syncthreads();
-          int wb = base;
-          for (int w = 0; w < (tid >> 6); ++w) wb += __float_as_int(res_v[w]);
-          if (t < n_tok) apos[t] = ap ? wb + before : -1;
-          for (int w = 0; w < kChainWaves; ++w) base += __float_as_int(res_v[w]);
-          __syncthreads();
-        }
-      }
-      if (tid < ntk) res_i[tid] = apos[t0 + tid];
-      __syncthreads();
+      const __amdgpu_buffer_rsrc_t akr = l2_rsrc(L.gate_appends ? gk_of(i) : pk_of(i), rowb);
+      const __amdgpu_buffer_rsrc_t avr = l2_rsrc(gv_of(i), rowb);
 #pragma unroll
       for (int it = 0; it < IT; ++it) {
-        const int lt = (tid + it * kChainThreads) / GL;
-        const bool valid = lt < ntk && res_i[lt] >= 0;
+        const int lt = it * RPP + sub;
         const int tl = lt < ntk ? t0 + lt : 0;  // token of this lane (token 0 when idle)
-        float k[8], v[8];
-        if (L.gate_appends) {
-          unpack8(*reinterpret_cast<const uint4 *>(&op_r[lt * STR + part * 8]), k);
-          unpack8(l2_ld16(l2_rsrc(gvb + rb * D, int64_t(n_tok) * D * 2), (tl * D + part * 8) * 2), v);
-        } else {
-          unpack8(*reinterpret_cast<const uint4 *>(&op_n[lt * STR + part * 8]), k);
-          load8(v_row + (tb + tl) * src.v_st + part * 8, v);
-        }
-        const float vlen = row_norm8<D>(v);
-        float ka[8], va[8];
-        attn_rows<D>(k, v, vlen, part, L, ln_w, ln_b, ka, va);
-        if (valid) {
-          const int64_t slot = sb + res_i[lt];
-          const int64_t so = (srow + slot) * D + part * 8;
-          store8(s_k + so, k);
-          store8(s_v + so, v);
-          if (part == 0) s_vlen[srow + slot] = vlen;
-          const int64_t ao = (int64_t(row) * cur.cap + slot) * D + part * 8;
-          store8(cur.k + ao, ka);
-          store8(cur.v + ao, va);
+        const bool valid = lt < ntk && apos[tl] >= 0;
+        if (__any(valid)) {
+          float k[8], v[8];
+          unpack8(l2_ld16(akr, (tl * D + part * 8) * 2), k);
+          if (L.gate_appends)
+            unpack8(l2_ld16(avr, (tl * D + part * 8) * 2), v);
+          else
+            load8(v_row + (tb + tl) * src.v_st + part * 8, v);
+          const float vlen = row_norm8<D>(v);
+          float ka[8], va[8];
+          attn_rows<D>(k, v, vlen, part, L, ln_w, ln_b, ka, va);
+          if (valid) {
+            const int64_t slot = sb + apos[tl];
+            const int64_t so = (srow + slot) * D + part * 8;
+            store8(s_k + so, k);
+            store8(s_v + so, v);
+            if (part == 0) s_vlen[srow + slot] = vlen;
+            store8(cur_k + slot * D + part * 8, ka);
+            store8(cur_v + slot * D + part * 8, va);
+          }
         }
       }
       KVM_TS_A(4);
       arrive();
+      // The next update's raw tokens while the group waits (loads return in
+      // order: anywhere else the loads behind them would wait for memory).
+      if (more) load_raw(i + 1, rt);
       if (!wait()) return;
+      load_own(cur_k, sb, s_after);
+      __syncthreads();
       KVM_TS_A(5);
+    } else {
+      load_bx(gk_of(i), tg0);
+      if (more) load_raw(i + 1, rt);
     }
 
-    // ---- route (model/kvm_fp32_routing_reference.py:30-34); the next
-    // update's raw tokens are loaded behind the scan's slot rows.
-    const bool more = i + 1 < list.count;
-    scan_slots<D, false>(op_r, cur_k, protect, s_after, ntk, red_v, red_i, res_v, res_i,
-                         [&]() __attribute__((always_inline)) {
-                           if (more) load_raw(i + 1, rt);
-                         });
+    // ---- route, then the next update's prep: with its rows stored before
+    // this update's routes are published, no barrier ends the update.
+    scan(std::false_type{}, gk_of(i), cur_k, protect, s_after);
     KVM_TS_A(6);
-    if (tid < ntk) {
-      const int t = t0 + tid;
-      const bool app = na > 0 && tok_a[t] != 0;
-      cs.route[rb + t] = app ? -1 : res_i[tid];
-      if (alog) alog[t] = app ? 1 : 0;
-      if (rlog) rlog[t] = app ? sb + apos[t] : res_i[tid];
+    if (more) prep(i + 1, rt);
+    __syncthreads();
+    uint2 *const part_row = cs.part + int64_t(i & 1) * rows * n_tok * G + rb * G;
+    for (int t = tid; t < n_tok; t += kChainThreads) {
+      uint64_t key = 0;
+      for (int x = 0; x < nsg; ++x) {
+        const uint64_t o = red[x * ntg * 64 + t];
+        key = o > key ? o : key;
+      }
+      part_row[t * G + member] = make_uint2(uint32_t(key >> 32), uint32_t(key));
     }
     KVM_TS_A(7);
     arrive();
     if (!wait()) return;
     KVM_TS_A(8);
 
-    // ---- merge + refresh (model/kvm_mixer.py:329-335) of my slots
-    const int spm = (s_after + G - 1) / G;
-    const int j0 = member * spm;
-    const int nsl = max(0, min(s_after, j0 + spm) - j0);
-    const __amdgpu_buffer_rsrc_t skr = l2_rsrc(s_k + srow * D, st.capacity * D * 2);
-    const __amdgpu_buffer_rsrc_t svr = l2_rsrc(s_v + srow * D, st.capacity * D * 2);
-    const __amdgpu_buffer_rsrc_t slr = l2_rsrc(s_vlen + srow, st.capacity * 4);
-    const __amdgpu_buffer_rsrc_t gkr = l2_rsrc(gkb + rb * D, int64_t(n_tok) * D * 2);
-    const __amdgpu_buffer_rsrc_t gvr = l2_rsrc(gvb + rb * D, int64_t(n_tok) * D * 2);
-    const __amdgpu_buffer_rsrc_t rr = l2_rsrc(cs.route + rb, int64_t(n_tok) * 4);
-    // Current sums and vlen of the first two slot passes (independent of the
-    // routes; rows past the state read zero and are not stored).
-    auto ld_state = [&](int local, uint4 &kk, uint4 &vv, float &ll) __attribute__((always_inline)) {
-      const int j = j0 + local;
-      kk = l2_ld16(skr, (j * D + part * 8) * 2);
-      vv = l2_ld16(svr, (j * D + part * 8) * 2);
-      ll = __uint_as_float(l2_ld4(slr, j * 4));
-    };
-    uint4 k0, v0, k1, v1;
-    float l0, l1;
-    ld_state(tid / GL, k0, v0, l0);
-    ld_state(RPP + tid / GL, k1, v1, l1);
-
-    for (int e = tid; e < nsl; e += kChainThreads) {
-      cnt[e] = 0;
-      fill[e] = 0;
+    // ---- the tokens of each of my slots, in token order: ballots rank the
+    // tokens of 64, counts per 64 tokens and slot place them.
+    const __amdgpu_buffer_rsrc_t pr = l2_rsrc(part_row, int64_t(n_tok) * G * 8);
+    const int nvw = (n_tok + 63) >> 6;
+    const int nblk = (s_after + 15) >> 4;
+    const int nown = member < nblk ? ((nblk - 1 - member) / G + 1) * 16 : 0;  // my local slots in use
+    for (int e = tid; e < nvw * own_cap; e += kChainThreads) wsc[e] = 0;
+    constexpr int NT = 2;  // tokens per thread (n_tok <= 1024)
+    int loc[NT], rank[NT];
+    uint64_t pkey[NT];
+#pragma unroll
+    for (int x = 0; x < NT; ++x) {
+      const int t = x * kChainThreads + tid;
+      pkey[x] = 0;
+      if (t < n_tok)
+      {
+        uint4 p4[G / 2];
+#pragma unroll
+        for (int m = 0; m < G / 2; ++m) p4[m] = l2_ld16(pr, (t * G + 2 * m) * 8);
+#pragma unroll
+        for (int m = 0; m < G / 2; ++m) {
+          const uint64_t a0 = (uint64_t(p4[m].x) << 32) | p4[m].y, a1 = (uint64_t(p4[m].z) << 32) | p4[m].w;
+          pkey[x] = a0 > pkey[x] ? a0 : pkey[x];
+          pkey[x] = a1 > pkey[x] ? a1 : pkey[x];
+        }
+      }
+    }
+    __syncthreads();  // wsc is cleared
+#pragma unroll
+    for (int x = 0; x < NT; ++x) {
+      const int t = x * kChainThreads + tid;
+      loc[x] = -1;
+      if (x * kChainThreads < n_tok) {
+        const int slot = route_key_slot(pkey[x]);
+        const bool app = na > 0 && t < n_tok && apos[t] >= 0;
+        if (t >= t0 && t < t0 + ntk) {  // each member logs its own tokens
+          if (alog) alog[t] = app ? 1 : 0;
+          if (rlog) rlog[t] = app ? sb + apos[t] : slot;
+        }
+        const bool mine = slot >= 0 && !app && (slot >> 4) % G == member;
+        const int l = mine ? (((slot >> 4) / G) << 4) | (slot & 15) : 0;
+        uint64_t eq = __ballot(mine);
+        for (int bit = 0; (1 << bit) < own_cap; ++bit) {
+          const uint64_t m = __ballot(mine && ((l >> bit) & 1));
+          eq &= ((l >> bit) & 1) ? m : ~m;
+        }
+        rank[x] = int(__builtin_amdgcn_mbcnt_hi(uint32_t(eq >> 32), __builtin_amdgcn_mbcnt_lo(uint32_t(eq), 0u)));
+        if (mine) loc[x] = l;
+        if (mine && rank[x] == 0) wsc[(x * kChainWaves + wave) * own_cap + l] = uint16_t(__popcll(eq));
+      }
     }
     __syncthreads();
-    for (int t = tid; t < n_tok; t += kChainThreads) {
-      const int r = int(l2_ld4(rr, t * 4));
-      const int lr = (r >= j0 && r < j0 + nsl) ? r - j0 : -1;
-      mr[t] = lr;
-      if (lr >= 0) atomicAdd(&cnt[lr], 1);
-    }
-    __syncthreads();
-    // Exclusive prefix of the slot counts on one wave.
-    if (tid < 64) {
-      const int per = (nsl + 63) >> 6;
-      const int e0 = tid * per;
-      int sum = 0;
-      for (int e = 0; e < per; ++e)
-        if (e0 + e < nsl) sum += cnt[e0 + e];
-      int incl = sum;
+    // Exclusive prefix: over the token groups of each slot's counts (in
+    // place), then over the slots, kChainThreads of them at a time.
+    for (int e0 = 0, run = 0; e0 < nown; e0 += kChainThreads) {
+      const int e = e0 + tid;
+      int tot = 0;
+      if (e < nown)
+        for (int w = 0; w < nvw; ++w) {
+          const int n = wsc[w * own_cap + e];
+          wsc[w * own_cap + e] = uint16_t(tot);
+          tot += n;
+        }
+      int incl = tot;
 #pragma unroll
       for (int o = 1; o < 64; o <<= 1) {
         const int y = __shfl_up(incl, o);
-        if (tid >= o) incl += y;
+        if (lane >= o) incl += y;
       }
-      int run = incl - sum;
-      for (int e = 0; e < per; ++e)
-        if (e0 + e < nsl) {
-          off[e0 + e] = run;
-          run += cnt[e0 + e];
-        }
-    }
-    __syncthreads();
-    for (int t = tid; t < n_tok; t += kChainThreads) {
-      const int lr = mr[t];
-      if (lr >= 0) lst[off[lr] + atomicAdd(&fill[lr], 1)] = t;
-    }
-    __syncthreads();
-    // Each slot's list in token order (rank sort), so the fp32 sums run in
-    // token order whatever order the LDS atomics placed them in.
-    for (int base = 0; base < nsl; base += RPP) {
-      const int local = base + tid / GL;
-      if (local < nsl) {
-        const int n = cnt[local], o = off[local];
-        for (int e = part; e < n; e += GL) {
-          const int x = lst[o + e];
-          int r = 0;
-          for (int f = 0; f < n; ++f) r += lst[o + f] < x;
-          sorted[o + r] = x;
-        }
+      if (lane == 63) wtot[wave] = incl;
+      __syncthreads();
+      int base = run + incl - tot;
+#pragma unroll
+      for (int w = 0; w < kChainWaves; ++w) {
+        base += w < wave ? wtot[w] : 0;
+        run += wtot[w];
       }
+      if (e < nown) {
+        off[e] = uint16_t(base);
+        cnt[e] = uint16_t(tot);
+      }
+      __syncthreads();
     }
+#pragma unroll
+    for (int x = 0; x < NT; ++x)
+      if (x * kChainThreads < n_tok && loc[x] >= 0)
+        sorted[off[loc[x]] + wsc[(x * kChainWaves + wave) * own_cap + loc[x]] + rank[x]] =
+            uint16_t(x * kChainThreads + tid);
     __syncthreads();
     KVM_TS_A(9);
-    auto merge_slot = [&](int local, const uint4 &k_raw, const uint4 &v_raw,
-                          float vlen) __attribute__((always_inline)) {
-      const bool valid = local < nsl;
-      const int j = j0 + (valid ? local : 0);
-      const int n = valid ? cnt[local] : 0;
-      const int o = valid ? off[local] : 0;
-      float sk[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-      float sv[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-      for (int i0 = 0; i0 < n; i0 += 4) {
-        uint4 xk[4], xv[4];
+
+    // ---- merge + refresh (model/kvm_mixer.py:329-335) of my slots.  A slot
+    // that no token was routed to keeps its attention rows: where none of a
+    // wave's rows changed (most, once the slots outnumber the tokens) they
+    // are copied, keys from LDS and values from the snapshot before.
+    const __amdgpu_buffer_rsrc_t skr = l2_rsrc(s_k + srow * D, st.capacity * D * 2);
+    const __amdgpu_buffer_rsrc_t svr = l2_rsrc(s_v + srow * D, st.capacity * D * 2);
+    const __amdgpu_buffer_rsrc_t slr = l2_rsrc(s_vlen + srow, st.capacity * 4);
+    const __amdgpu_buffer_rsrc_t gkr = l2_rsrc(gk_of(i), rowb);
+    const __amdgpu_buffer_rsrc_t gvr = l2_rsrc(gv_of(i), rowb);
+    const __amdgpu_buffer_rsrc_t ckr = l2_rsrc(cur_k, int64_t(s_after) * D * 2);
+    const __amdgpu_buffer_rsrc_t cvr = l2_rsrc(cur_v, int64_t(s_after) * D * 2);
+    const __amdgpu_buffer_rsrc_t nk = l2_rsrc(nxt.k + int64_t(row) * nxt.cap * D, int64_t(s_after) * D * 2);
+    const __amdgpu_buffer_rsrc_t nv = l2_rsrc(nxt.v + int64_t(row) * nxt.cap * D, int64_t(s_after) * D * 2);
+    constexpr int MP = 2;  // slot passes whose loads are in flight together
+    for (int l0 = 0; l0 < nown; l0 += MP * RPP) {
+      uint4 kk[MP], vv[MP];
+      float vl[MP];
+      int n[MP], jj[MP];
+      bool any[MP];  // uniform: some slot of my wave's rows changed
 #pragma unroll
-        for (int w = 0; w < 4; ++w) {
-          if (i0 + w < n) {
-            const int to = (sorted[o + i0 + w] * D + part * 8) * 2;
-            xk[w] = l2_ld16(gkr, to);
-            xv[w] = l2_ld16(gvr, to);
-          }
+      for (int x = 0; x < MP; ++x) {
+        const int l = l0 + x * RPP + sub;
+        jj[x] = own_local_to_slot(l, G, member);  // rows at or past s_after lie past the resources
+        n[x] = l < nown && jj[x] < s_after ? cnt[l] : 0;
+        any[x] = __any(n[x] > 0);
+        const int o = (jj[x] * D + part * 8) * 2;
+        if (any[x]) {
+          kk[x] = l2_ld16(skr, o);
+          vv[x] = l2_ld16(svr, o);
+          vl[x] = __uint_as_float(l2_ld4(slr, jj[x] * 4));
+        } else {
+          vv[x] = l2_ld16(cvr, o);
+          if (l < OWNL)
+            kk[x] = *reinterpret_cast<const uint4 *>(&own_k[l * STR + part * 8]);
+          else
+            kk[x] = l2_ld16(ckr, o);
         }
+      }
 #pragma unroll
-        for (int w = 0; w < 4; ++w) {
-          if (i0 + w < n) {
-            float fk[8], fv[8];
-            unpack8(xk[w], fk);
-            unpack8(xv[w], fv);
+      for (int x = 0; x < MP; ++x) {
+        const int l = l0 + x * RPP + sub;
+        if (any[x]) {
+          float sk[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+          float sv[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+          const int o = n[x] > 0 ? off[l] : 0;
+          for (int i0 = 0; i0 < n[x]; i0 += 4) {
+            uint4 xk[4], xv[4];
 #pragma unroll
-            for (int e = 0; e < 8; ++e) {
-              sk[e] += fk[e];
-              sv[e] += fv[e];
+            for (int w = 0; w < 4; ++w) {
+              if (i0 + w < n[x]) {
+                const int to = (int(sorted[o + i0 + w]) * D + part * 8) * 2;
+                xk[w] = l2_ld16(gkr, to);
+                xv[w] = l2_ld16(gvr, to);
+              }
+            }
+#pragma unroll
+            for (int w = 0; w < 4; ++w) {
+              if (i0 + w < n[x]) {
+                float fk[8], fv[8];
+                unpack8(xk[w], fk);
+                unpack8(xv[w], fv);
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                  sk[e] += fk[e];
+                  sv[e] += fv[e];
+                }
+              }
             }
           }
-        }
-      }
-      float k[8], v[8];
-      unpack8(k_raw, k);
-      unpack8(v_raw, v);
-      const int64_t so = (srow + j) * D + part * 8;
-      if (n > 0) {
+          float k[8], v[8];
+          unpack8(kk[x], k);
+          unpack8(vv[x], v);
+          if (n[x] > 0) {  // state = bf16(state + bf16(sum))
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          k[e] = rbf(k[e] + rbf(sk[e]));
-          v[e] = rbf(v[e] + rbf(sv[e]));
+            for (int e = 0; e < 8; ++e) {
+              k[e] = rbf(k[e] + rbf(sk[e]));
+              v[e] = rbf(v[e] + rbf(sv[e]));
+            }
+            const int64_t so = (srow + jj[x]) * D + part * 8;
+            store8(s_k + so, k);
+            store8(s_v + so, v);
+          }
+          float ka[8], va[8];
+          attn_rows<D>(k, v, vl[x], part, L, ln_w, ln_b, ka, va);
+          kk[x] = pack8(ka);
+          vv[x] = pack8(va);
+          if (l < nown && l < OWNL) *reinterpret_cast<uint4 *>(&own_k[l * STR + part * 8]) = kk[x];
         }
-        if (valid) {
-          store8(s_k + so, k);
-          store8(s_v + so, v);
-        }
+        // Streamed: the attention kernel reads the snapshot much later.
+        const uint32_t so = uint32_t((jj[x] * D + part * 8) * 2);
+        st16<kPolicyNT>(nk, so, kk[x]);
+        st16<kPolicyNT>(nv, so, vv[x]);
       }
-      float ka[8], va[8];
-      attn_rows<D>(k, v, vlen, part, L, ln_w, ln_b, ka, va);
-      if (valid) {
-        const int64_t ao = (int64_t(row) * nxt.cap + j) * D + part * 8;
-        store8(nxt.k + ao, ka);
-        store8(nxt.v + ao, va);
-      }
-    };
-    for (int base = 0; base < nsl; base += 2 * RPP) {
-      if (base > 0) {
-        ld_state(base + tid / GL, k0, v0, l0);
-        ld_state(base + RPP + tid / GL, k1, v1, l1);
-      }
-      merge_slot(base + tid / GL, k0, v0, l0);
-      if (base + RPP < nsl) merge_slot(base + RPP + tid / GL, k1, v1, l1);
     }
     KVM_TS_A(10);
-
-    // ---- next update's prep while the other members finish this merge.
-    if (more) {
-      arrive();
-      prep(i + 1, rt);
-      KVM_TS_A(11);
-      if (!wait()) return;
-      KVM_TS_A(12);
-    }
+    // My slots' new rows before the next scan: in LDS, and for slots past it
+    // in the snapshot.
+    if (own_cap > OWNL) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    KVM_TS_A(11);
+    KVM_TS_A(12);
   }
 }
 
@@ -856,9 +909,6 @@ constexpr int kOwnMax = 128;      // owned slots per member at most (8 blocks of
 constexpr int kTokWave = 64;      // tokens per wave in route(p)
 constexpr int kFixedMaxTok = kChainWaves * kTokWave;  // == kChainThreads: one token per thread
 
-__device__ __forceinline__ int own_local_to_slot(int l, int G, int m) {
-  return (((l >> 4) * G + m) << 4) | (l & 15);
-}
 
 // GM: the group size G (8 or 16); OWN: owned slots per member the LDS holds
 // (64, or 128 for states of up to 1024 slots at G = 8).
@@ -1942,26 +1992,31 @@ bool chain_plan(const kvm_layer &L, int64_t n_tok, int64_t max_slots, ChainPlan 
   const int64_t limit = std::min<int64_t>(kChainMaxWorkgroups, cus);
   const int64_t rows = L.batch * L.kv_heads;
   const int64_t groups = (rows + 7) / 8 * 8;
-  int G = groups * 16 <= limit ? 16 : 8;
-  // More rows than one launch keeps resident: consecutive launches over
-  // batches of rows (launch_chain).
-  const int64_t tpw = ((n_tok + G - 1) / G + 15) / 16 * 16;
-  if (tpw > kChainTok || limit / G < 8 || n_tok < 1) return false;
-  p->fixed = false;
-  p->G = G;
-  p->limit = int(limit);
-  p->rows = int(rows);
-  p->head_dim = int(L.head_dim);
-  p->tpw = int(tpw);
-  p->spm_max = int((max_slots + G - 1) / G);
-  // ints of the lists, then the append selection's 8-byte keys (a power of
-  // two of them) after one int of alignment padding.
-  int64_t npow = 1;
-  while (npow < n_tok) npow <<= 1;
-  const int64_t dyn = (4 * n_tok + 3 * int64_t(p->spm_max) + 1) * 4 + npow * 8;
-  if (dyn > 48 * 1024) return false;
-  p->dyn_lds = size_t(dyn);
-  return true;
+  // Members per row of the appending chain: 16 while every row fits one
+  // launch, 8 up to what that keeps resident, then 4 (each launch holds twice
+  // the rows of 8 members and takes less than twice as long: us per update for
+  // all rows with 8 / 4 members, 48 rows of 1425 slots 57.0 / 38.8, 64 rows of
+  // 872 64-wide slots 38.3 / 23.6, 256 rows of 868 slots, C 128, 190 / 116).
+  // More rows than a launch keeps resident: consecutive launches over batches
+  // of rows (launch_chain).
+  for (int G : {16, 4, 8}) {
+    if ((G == 16 && groups * 16 > limit) || (G == 4 && groups * 8 <= limit)) continue;
+    const int64_t tpw = ((n_tok + G - 1) / G + 15) / 16 * 16;
+    const int64_t own_cap = ((max_slots + 15) / 16 + G - 1) / G * 16;
+    if (tpw > kChainTok || limit / G < 8 || n_tok < 1 || max_slots > 32768) continue;
+    const int64_t dyn = append_lds_bytes(int(n_tok), int(own_cap));
+    if (dyn > kAppendDynLds) continue;
+    p->fixed = false;
+    p->G = G;
+    p->limit = int(limit);
+    p->rows = int(rows);
+    p->head_dim = int(L.head_dim);
+    p->tpw = int(tpw);
+    p->own_cap = int(own_cap);
+    p->dyn_lds = size_t(dyn);
+    return true;
+  }
+  return false;
 }
 
 namespace {
@@ -2016,8 +2071,8 @@ int64_t chain_scratch_bytes(const kvm_layer &L, int64_t n_tok) {
   const size_t tok = size_t(L.batch * L.kv_heads) * size_t(n_tok);
   auto a256 = [](size_t x) { return (x + 255) & ~size_t(255); };
   // four merge buffers of keys, four of values (buffer b at gk + b * rows * n_tok * D),
-  // routes, novelty, two sets of per-member maxima (up to 16 members), counters
-  return int64_t(2 * a256(4 * tok * size_t(L.head_dim) * 2) + 2 * a256(tok * 4) +
+  // per-member novelties and two sets of route maxima (up to 16 members), counters
+  return int64_t(2 * a256(4 * tok * size_t(L.head_dim) * 2) + a256(tok * 16 * 4) +
                  a256(2 * tok * 16 * 8) +
                  a256(size_t(kChainMaxWorkgroups) * kCounterStride * 4 + 256));
 }
@@ -2027,14 +2082,13 @@ ChainScratch carve_chain_scratch(void *base, const kvm_layer &L, int64_t n_tok) 
   auto a256 = [](size_t x) { return (x + 255) & ~size_t(255); };
   unsigned char *p = static_cast<unsigned char *>(base);
   ChainScratch c;
-  const size_t kb = tok * size_t(L.head_dim) * 2, ib = a256(tok * 4);
+  const size_t kb = tok * size_t(L.head_dim) * 2, ib = a256(tok * 16 * 4);
   const size_t kb4 = a256(4 * kb), pb = a256(2 * tok * 16 * 8);
   c.gk = reinterpret_cast<uint16_t *>(p);
   c.gv = reinterpret_cast<uint16_t *>(p + kb4);
-  c.route = reinterpret_cast<int32_t *>(p + 2 * kb4);
-  c.nov = reinterpret_cast<float *>(p + 2 * kb4 + ib);
-  c.part = reinterpret_cast<uint2 *>(p + 2 * kb4 + 2 * ib);
-  c.bar = reinterpret_cast<unsigned *>(p + 2 * kb4 + 2 * ib + pb);
+  c.nov = reinterpret_cast<float *>(p + 2 * kb4);
+  c.part = reinterpret_cast<uint2 *>(p + 2 * kb4 + ib);
+  c.bar = reinterpret_cast<unsigned *>(p + 2 * kb4 + ib + pb);
   c.abort_flag = c.bar + size_t(kChainMaxWorkgroups) * kCounterStride;
   c.status = nullptr;  // set by the caller
   c.max_polls = kChainDefaultPolls;
@@ -2096,12 +2150,24 @@ hipError_t launch_chain(const kvm_layer &L, const kvm_seq &src, int64_t n_tok,
       }
 #undef KVM_FIXED_D
 #undef KVM_FIXED
-    } else if (L.head_dim == 128) {
-      hipLaunchKernelGGL(k_chain<128>, grid, blk, p.dyn_lds, stream, L, src, int(n_tok), st, snaps, list, cs,
-                         rows, row0, nrows, G, p.tpw, p.spm_max, route_log, append_log, log_stride);
     } else {
-      hipLaunchKernelGGL(k_chain<64>, grid, blk, p.dyn_lds, stream, L, src, int(n_tok), st, snaps, list, cs,
-                         rows, row0, nrows, G, p.tpw, p.spm_max, route_log, append_log, log_stride);
+#define KVM_APPEND(DD, GG)                                                                                   \
+  hipLaunchKernelGGL((k_chain<DD, GG>), grid, blk, p.dyn_lds, stream, L, src, int(n_tok), st, snaps, list, cs, \
+                     rows, row0, nrows, p.tpw, p.own_cap, route_log, append_log, log_stride)
+#define KVM_APPEND_D(DD)   \
+  if (G == 16)             \
+    KVM_APPEND(DD, 16);    \
+  else if (G == 8)         \
+    KVM_APPEND(DD, 8);     \
+  else                     \
+    KVM_APPEND(DD, 4)
+      if (L.head_dim == 128) {
+        KVM_APPEND_D(128);
+      } else {
+        KVM_APPEND_D(64);
+      }
+#undef KVM_APPEND_D
+#undef KVM_APPEND
     }
     e = hipGetLastError();
     if (e != hipSuccess) return e;

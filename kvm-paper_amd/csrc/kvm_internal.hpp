@@ -102,10 +102,9 @@ struct SnapRing {
   int64_t cap;     // slots per row
 };
 struct ChainScratch {
-  uint16_t *gk;          // merge keys   bf16 [3][rows, n_tok, D] (rotating over updates)
-  uint16_t *gv;          // merge values bf16 [3][rows, n_tok, D]
-  int32_t *route;        // merge slot of each token, -1 if appended [rows, n_tok]
-  float *nov;            // novelty of each token [rows, n_tok]
+  uint16_t *gk;          // merge keys   bf16 [4][rows, n_tok, D] (rotating over updates)
+  uint16_t *gv;          // merge values bf16 [4][rows, n_tok, D]
+  float *nov;            // per-member novelties of each token [rows, n_tok, G]
   uint2 *part;           // per-member route maxima as route keys {mono(score), tag << 16 | (0xffff - slot)} [2][rows, n_tok, G]
   unsigned *bar;         // group barrier counters
   unsigned *abort_flag;  // set when a group wait timed out (cleared per launch)
@@ -116,7 +115,7 @@ struct ChainPlan {
   bool fixed;     // slot-owner routing (no appends in the batch)
   int G;          // workgroups per row
   int tpw;        // tokens per workgroup (multiple of 16, <= 64)
-  int spm_max;    // slots per workgroup at max_slots
+  int own_cap;    // owned slots per member at max_slots (whole blocks of 16)
   int limit;      // workgroups a launch keeps resident
   int rows;       // rows of the call
   int head_dim;

@@ -1040,3 +1040,34 @@ def test_chain_many_rows_matches_per_update_kernels(lib, monkeypatch, B, Hkv, Tn
     assert res["1"]["plan"].n_updates > 0
     for key in ("route_log", "append_log", "out", "state_k", "state_v", "state_vlen", "state_k_attn", "state_v_attn"):
         assert torch.equal(res["1"][key], res["0"][key]), key
+
+
+@pytest.mark.parametrize("B,Hkv,Tn,D,C,mode,round_down", [
+    (5, 8, 12000, 128, 256, "power_law", 1),     # four members per row; more own slots than LDS rows
+    (1, 2, 6000, 128, 1000, "power_law", 1),     # 16 members, 16 token groups, ragged chunk
+    (1, 3, 3000, 64, 40, "kvm_saturation", 16),  # one token group; updates without appends in between
+    (3, 8, 3001, 64, 130, "kvm_saturation", 1),  # eight members, ragged chunk
+])
+def test_appending_chain_matches_per_update_kernels(lib, monkeypatch, B, Hkv, Tn, D, C, mode, round_down):
+    """The appending chain's group sizes, token groups and slot storage at
+    their edges: append sets, routes, state and outputs must equal the
+    per-update kernels bit for bit."""
+    T.log(f"[chain-append] B{B} Hkv{Hkv} T{Tn} D{D} C{C} {mode} round_down {round_down}")
+    cfg = T.mixer_config(Hkv, Hkv, D, C, mode=mode, sink=1, min_len=1, n_max=-(-4096 // C), factor=16.0, sat_n=1024,
+                         round_down=round_down)
+    gen = torch.Generator().manual_seed(3)
+    ln_w = (1 + 0.1 * torch.randn(D, generator=gen)).bfloat16()
+    ln_b = (0.1 * torch.randn(D, generator=gen)).bfloat16()
+    m = T.make_mixer(cfg, ln_w, ln_b, torch.ones(Hkv), torch.ones(Hkv))
+    q, k, v, g = (t.to(DEV) for t in _random_inputs(B, Hkv, Hkv, Tn, D, 37))
+    res = {}
+    for chain in ("1", "0"):
+        monkeypatch.setenv("KVM_AMD_CHAIN", chain)
+        with torch.no_grad():
+            res[chain] = m.prefill_raw(q, k, v, g, route_log=True)
+        torch.cuda.synchronize()
+    plan = res["1"]["plan"]
+    assert sum(plan.upd_n_append) > 0
+    T.log(f"[chain-append] {plan.n_updates} updates, {plan.initial_state_len} -> {plan.final_state_len} slots")
+    for key in ("append_log", "route_log", "out", "state_k", "state_v", "state_vlen", "state_k_attn", "state_v_attn"):
+        assert torch.equal(res["1"][key], res["0"][key]), key
