@@ -252,6 +252,10 @@ typedef struct kvm_state_bwd_desc {
 
 int64_t kvm_state_backward_workspace_bytes(const kvm_state_bwd_desc *d);
 int kvm_state_backward(const kvm_state_bwd_desc *d, void *stream);
+/* The same with the sums rounded once into dk_out / dv_out (bf16 [B, Hkv,
+ * seq_len, head_dim], 16-byte aligned), every token's row; dk / dv are only
+ * read.  The updates' chunks must follow each other without gaps. */
+int kvm_state_backward_rounded(const kvm_state_bwd_desc *d, void *dk_out, void *dv_out, void *stream);
 
 /* The mixer's pre-boundary elementwise work on the q/k/v projections, for
  * one layer (model/value_residual_mixin.py:173-237 calc_qkv and

@@ -219,6 +219,7 @@ struct StateBwdArgs {
   const float *d_snap_k, *d_snap_v;
   float *dk, *dv, *dgate;
   float *d_ln;                            // [2, D]
+  uint16_t *dk16, *dv16;                  // optional bf16 [rows, T, D]: the sums go here, dk / dv are only read
 };
 // Per-update schedule, passed by value as a kernel argument (3 KiB).
 struct UpdTable {
@@ -226,9 +227,10 @@ struct UpdTable {
   int32_t state_before[kMaxChunksPerLaunch];
   int32_t n_append[kMaxChunksPerLaunch];
 };
-int64_t state_bwd_workspace_bytes(int64_t head_dim, int64_t rows, int64_t max_state_len);
+int64_t state_bwd_workspace_bytes(int64_t head_dim, int64_t rows, int64_t max_state_len, int64_t n_updates,
+                                  int64_t chunk_len);
 int64_t state_bwd_max_chunk();
-// part: the per-workgroup LayerNorm partials (the workspace).
+// part: the workspace (per-workgroup LayerNorm partials, grouped route entries).
 hipError_t launch_state_backward(const StateBwdArgs &a, const UpdTable &sched, float *part,
                                  hipStream_t stream);
 

@@ -46,7 +46,7 @@ namespace {
 constexpr int kThreads = 64;  // one wave per workgroup: the per-update compaction needs no barrier
 constexpr int kMaxChunk = 4096;
 constexpr float kNormEps = 1e-12f;  // torch.nn.functional.normalize
-constexpr int kPf = 8;              // route entries per lane loaded one update ahead
+constexpr int kSortGroups = 4096;   // slot groups that k_route_sort places at a time
 
 __device__ __forceinline__ void load8f(const float *p, float (&x)[8]) {
   const float4 a = *reinterpret_cast<const float4 *>(p), b = *reinterpret_cast<const float4 *>(p + 4);
@@ -194,18 +194,95 @@ __device__ __forceinline__ void tok_backward(const StateBwdArgs &A, const Tok &x
     if (part * 8 + e >= A.L.rope_partial_dim) dk[e] += x.r * (dxh[e] - m1 - x.xh[e] * m2);
     dv[e] += (gv ? dxv[e] * x.g : dxv[e]) + dvl[e];
   }
-  store8f(A.dk + o, dk);
-  store8f(A.dv + o, dv);
+  if (A.dk16) {  // the caller takes the rounded sums instead
+    store8(A.dk16 + o, dk);
+    store8(A.dv16 + o, dv);
+  } else {
+    store8f(A.dk + o, dk);
+    store8f(A.dv + o, dv);
+  }
   if (part == 0) A.dgate[tok_row] = dg;
 }
 
+// Groups the entries of every update by the workgroup that owns their slot
+// (RPW slots each), in token order within a group: entry
+// (token << 8) | (local slot << 1) | appended; group g of update u of a row is
+// ent[(u * rows + row) * C + off[g] .. off[g + 1]).  One wave per (update,
+// row): counts by LDS atomics, a prefix over the groups, and a stable
+// placement 64 tokens at a time (ballots over the group index).  The state
+// kernel used to compact the routes in every wave, in both scans: 17 % of its
+// instructions.
+template <int RPW>
+__global__ __launch_bounds__(kThreads) void k_route_sort(const int32_t *route, const int32_t *append, int rows, int C,
+                                                         int ngrp, int32_t *ent, int32_t *off) {
+  __shared__ int fill[kSortGroups];
+  const int lane = threadIdx.x;
+  const int64_t ur = int64_t(blockIdx.y) * rows + blockIdx.x;  // (update, row)
+  route += ur * C;
+  append += ur * C;
+  ent += ur * C;
+  off += ur * (ngrp + 1);
+  int base = 0;
+  for (int g0 = 0; g0 < ngrp; g0 += kSortGroups) {
+    const int ng = min(kSortGroups, ngrp - g0);
+    for (int g = lane; g < ng; g += kThreads) fill[g] = 0;
+    __syncthreads();
+    for (int t = lane; t < C; t += kThreads) {
+      const int g = route[t] / RPW - g0;
+      if (route[t] >= 0 && g >= 0 && g < ng) atomicAdd(&fill[g], 1);
+    }
+    __syncthreads();
+    for (int g1 = 0; g1 < ng; g1 += kThreads) {
+      const int g = g1 + lane, n = g < ng ? fill[g] : 0;
+      int incl = n;
+#pragma unroll
+      for (int o = 1; o < 64; o <<= 1) {
+        const int y = __shfl_up(incl, o);
+        if (lane >= o) incl += y;
+      }
+      if (g < ng) {
+        fill[g] = base + incl - n;
+        off[g0 + g] = base + incl - n;
+      }
+      base += __shfl(incl, 63);
+    }
+    __syncthreads();
+    for (int t0 = 0; t0 < C; t0 += kThreads) {
+      const int t = t0 + lane, r = t < C ? route[t] : -1, g = r / RPW - g0;
+      const bool hit = r >= 0 && g >= 0 && g < ng;
+      uint64_t eq = __ballot(hit);
+      if (eq == 0) continue;
+      for (int bit = 0; (1 << bit) < ng; ++bit) {
+        const uint64_t m = __ballot(hit && ((g >> bit) & 1));
+        eq &= ((g >> bit) & 1) ? m : ~m;
+      }
+      const int rank = int(__builtin_amdgcn_mbcnt_hi(uint32_t(eq >> 32), __builtin_amdgcn_mbcnt_lo(uint32_t(eq), 0u)));
+      const int at = hit ? fill[g] : 0;
+      __syncthreads();  // read before the group's first lane moves it on
+      if (hit) {
+        ent[at + rank] = (t << 8) | ((r % RPW) << 1) | (append[t] ? 1 : 0);
+        if (rank == 0) fill[g] = at + int(__popcll(eq));
+      }
+      __syncthreads();
+    }
+  }
+  if (lane == 0) off[ngrp] = base;
+}
+
+// Bound by VALU issue (the tokens' LayerNorms and chain rule, the slots'
+// local backward) and by memory: 2 waves per SIMD, so every load a batch
+// needs is issued a batch ahead, into the registers the batch before has
+// given up.  32 rows of 512 slots, 61 updates of 512 tokens: 1724 us with the
+// routes compacted in every wave and each batch's loads waited for, 1377 so
+// (plus 18 for k_route_sort), 1319 with the sums rounded to bf16 here (which
+// also takes two casts of dk / dv, 330 us, out of the training step).
 template <int D>
-__global__ __launch_bounds__(kThreads) void k_state_bwd(StateBwdArgs A, UpdTable U, float *__restrict__ dln_part) {
+__global__ __launch_bounds__(kThreads) void k_state_bwd(StateBwdArgs A, UpdTable U, const int32_t *__restrict__ ent,
+                                                        const int32_t *__restrict__ goff,
+                                                        float *__restrict__ dln_part) {
   constexpr int GL = D / 8;            // lanes per slot row (a lane group)
   constexpr int RPW = kThreads / GL;   // slot rows per workgroup = lane groups
-  // Tokens of the current update routed to this workgroup's slots, in token
-  // order: (token << 8) | (local slot << 1) | appended (dynamic LDS, chunk_len entries).
-  extern __shared__ int32_t lst[];
+  __shared__ int32_t span[kMaxChunksPerLaunch];  // my entries of each update: first << 16 | count
   __shared__ __attribute__((aligned(16))) float rows[RPW][2][D];  // token rows, one per lane group
   __shared__ __attribute__((aligned(16))) float accb[RPW][2][D];  // slot gradients (reverse scan)
   __shared__ float accl_s[RPW];
@@ -231,41 +308,22 @@ __global__ __launch_bounds__(kThreads) void k_state_bwd(StateBwdArgs A, UpdTable
   auto tb_of = [&](int u) { return U.token_begin[u]; };
   auto before_of = [&](int u) { return U.state_before[u]; };
   auto napp_of = [&](int u) { return U.n_append[u]; };
-  // Route / append entries of the first kPf * 64 tokens of an update are
-  // loaded one update ahead (in registers); the rest, if any, when used.
-  int pr[kPf], pa[kPf];
-  auto prefetch = [&](int u) {
-    if (u < 0 || u >= nu) return;
-    const int64_t o = (int64_t(u) * A.rows + row) * C;
-#pragma unroll
-    for (int it = 0; it < kPf; ++it) {
-      const int t = it * kThreads + tid;
-      pr[it] = t < C ? A.route_log[o + t] : -1;
-      pa[it] = t < C ? A.append_log[o + t] : 0;
-    }
+  for (int u = tid; u < nu; u += kThreads) {
+    const int64_t o = (int64_t(u) * A.rows + row) * (gridDim.x + 1) + blockIdx.x;
+    span[u] = (goff[o] << 16) | (goff[o + 1] - goff[o]);
+  }
+  __syncthreads();
+  auto count_of = [&](int u) { return u >= 0 && u < nu ? __builtin_amdgcn_readfirstlane(span[u]) & 0xffff : 0; };
+  // Entry i of update u (0 past its end, or when there is no such update).
+  auto entry_at = [&](int u, int i) {
+    if (u < 0 || u >= nu) return 0;
+    const int sp = __builtin_amdgcn_readfirstlane(span[u]);
+    return i < (sp & 0xffff) ? ent[(int64_t(u) * A.rows + row) * C + (sp >> 16) + i] : 0;
   };
-  // Ordered compaction of update u's routes onto [j0, j0 + RPW) (the first
-  // part from the prefetched registers); returns the list length (the same
-  // in every lane).
-  auto stage = [&](int u) {
-    const int64_t o = (int64_t(u) * A.rows + row) * C;
-    int n = 0;
-    __syncthreads();  // the previous list has been read
-    auto add = [&](int t, int r, int a) {
-      const bool hit = r >= j0 && r < j0 + RPW;
-      const uint64_t m = __ballot(hit);
-      if (hit) lst[n + __popcll(m & ((uint64_t(1) << lane) - 1))] = (t << 8) | ((r - j0) << 1) | (a ? 1 : 0);
-      n += __popcll(m);
-    };
-#pragma unroll
-    for (int it = 0; it < kPf; ++it) add(it * kThreads + tid, pr[it], pa[it]);
-    for (int t0 = kPf * kThreads; t0 < C; t0 += kThreads) {
-      const int t = t0 + tid;
-      add(t, t < C ? A.route_log[o + t] : -1, t < C ? A.append_log[o + t] : 0);
-    }
-    __syncthreads();  // the list is complete
-    return n;
-  };
+  // The first 64 entries of the present update and the next two, one per lane.
+  int32_t e_cur = 0, e_next = 0, e_far = 0;
+  // Entry i0 + my of the present update (from memory past the first 64).
+  auto cur_entry = [&](int u, int i0) { return i0 + RPW <= 64 ? __shfl(e_cur, i0 + my) : entry_at(u, i0 + my); };
   auto put_rows = [&](const float (&rk)[8], const float (&rv)[8]) {
     store8f(&rows[my][0][part * 8], rk);
     store8f(&rows[my][1][part * 8], rv);
@@ -285,23 +343,41 @@ __global__ __launch_bounds__(kThreads) void k_state_bwd(StateBwdArgs A, UpdTable
 #pragma unroll
     for (int e = 0; e < 8; ++e) sk[e] = sv[e] = 0.f;
   }
-  prefetch(0);
+  // `raw` holds the rows of the batch to come (token 0 of the row when there
+  // is none); a batch reloads it as soon as it has consumed it.
+  RawTok raw = fetch_tok(R, 0, part);
+  int32_t e_raw = 0;
+  auto fetch_first = [&](int u) {  // the first batch of update u, whose entries are e_next
+    e_raw = __shfl(e_next, my);
+    raw = fetch_tok(R, u >= 0 && u < nu ? tb_of(u) + (e_raw >> 8) : 0, part);
+  };
+  e_next = entry_at(0, lane);
+  e_far = entry_at(1, lane);
+  fetch_first(0);
   for (int u = 0; u < nu; ++u) {
-    const int n = stage(u);
-    prefetch(u + 1);
-    const int tb = tb_of(u);
+    e_cur = e_next;
+    e_next = e_far;
+    e_far = entry_at(u + 2, lane);
+    const int n = count_of(u);
     float dk[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f}, dv[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
     for (int i0 = 0; i0 < n; i0 += RPW) {
-      const int i = i0 + my;
-      const int e = i < n ? lst[i] : 0;
+      const int e = e_raw;
       Tok x;
-      make_tok<D>(A, fetch_tok(R, tb + (e >> 8), part), part, w, bb, x);
+      make_tok<D>(A, raw, part, w, bb, x);
+      __builtin_amdgcn_sched_barrier(0);
+      if (i0 + RPW < n) {  // uniform
+        e_raw = cur_entry(u, i0 + RPW);
+        raw = fetch_tok(R, tb_of(u) + (e_raw >> 8), part);
+      } else {
+        fetch_first(u + 1);
+      }
+      __builtin_amdgcn_sched_barrier(0);
       float rk[8], rv[8];
       tok_rows(A.L, x, (e & 1) ? kAppended : kMerged, rk, rv);
       put_rows(rk, rv);
       __syncthreads();
       for (int g = 0; g < RPW && i0 + g < n; ++g) {
-        const int eg = lst[i0 + g];
+        const int eg = __builtin_amdgcn_readlane(e, g * GL);
         if (((eg >> 1) & 127) != my) continue;
         float xk[8], xv[8];
         load8f(&rows[g][0][part * 8], xk);
@@ -323,6 +399,7 @@ __global__ __launch_bounds__(kThreads) void k_state_bwd(StateBwdArgs A, UpdTable
       }
       __syncthreads();  // rows is rewritten by the next batch
     }
+    if (n == 0) fetch_first(u + 1);
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
       sk[e] += dk[e];
@@ -344,8 +421,19 @@ __global__ __launch_bounds__(kThreads) void k_state_bwd(StateBwdArgs A, UpdTable
       load8f(A.d_snap_v + so, gv);
     }
   };
-  prefetch(nu - 1);
+  // A batch's rows of A.dk / A.dv (one writer per row, so they may be read
+  // ahead), given up by the batch before once it has stored its own.
+  float cdk[8], cdv[8];
+  auto fetch_grad = [&](int u) {  // of the batch in `raw`, of update u
+    const int64_t o = (rowT + (u >= 0 ? tb_of(u) + (e_raw >> 8) : 0)) * D + part * 8;
+    load8f(A.dk + o, cdk);
+    load8f(A.dv + o, cdv);
+  };
   load_snap(nu);
+  e_next = entry_at(nu - 1, lane);
+  e_far = entry_at(nu - 2, lane);
+  fetch_first(nu - 1);
+  fetch_grad(nu - 1);
   for (int s = nu; s >= 0; --s) {
     const int len = snap_len(s);
     if (j < len) {
@@ -394,39 +482,46 @@ __global__ __launch_bounds__(kThreads) void k_state_bwd(StateBwdArgs A, UpdTable
     // owning slot's gradient (published in accb), the owner subtracts the
     // merged rows in list order.
     const int u = s - 1;
-    const int n = stage(u);
-    prefetch(u - 1);
+    e_cur = e_next;
+    e_next = e_far;
+    e_far = entry_at(u - 2, lane);
+    const int n = count_of(u);
     load_snap(s - 1);  // used at the next step
-    const int tb = tb_of(u);
     store8f(&accb[my][0][part * 8], acck);
     store8f(&accb[my][1][part * 8], accv);
     if (part == 0) accl_s[my] = accl;
     __syncthreads();
     for (int i0 = 0; i0 < n; i0 += RPW) {
-      const int i = i0 + my;
-      const bool valid = i < n;
-      const int e = valid ? lst[i] : 0;
-      const int64_t t = tb + (e >> 8);
+      const int e = e_raw;
+      const bool valid = i0 + my < n;
+      const int64_t t = tb_of(u) + (e >> 8);
       const int ls = (e >> 1) & 127;
-      const RawTok raw = fetch_tok(R, t, part);
-      float cdk[8], cdv[8];  // the token's rows of A.dk / A.dv, loaded with its k / v
-      const int64_t o = (rowT + t) * D + part * 8;
-      load8f(A.dk + o, cdk);
-      load8f(A.dv + o, cdv);
       Tok x;
       make_tok<D>(A, raw, part, w, bb, x);
+      __builtin_amdgcn_sched_barrier(0);
+      const bool more = i0 + RPW < n;  // uniform
+      if (more) {
+        e_raw = cur_entry(u, i0 + RPW);
+        raw = fetch_tok(R, tb_of(u) + (e_raw >> 8), part);
+      } else {
+        fetch_first(u - 1);
+      }
+      __builtin_amdgcn_sched_barrier(0);
       float ak[8], av[8];
       load8f(&accb[ls][0][part * 8], ak);
       load8f(&accb[ls][1][part * 8], av);
       const bool app = (e & 1) != 0;
       if (valid) tok_backward<D>(A, x, app ? kAppended : kMerged, rowT + t, part, w, ak, av,
                                  app ? accl_s[ls] : 0.f, dlw, dlb, cdk, cdv);
+      __builtin_amdgcn_sched_barrier(0);
+      fetch_grad(more ? u : u - 1);
+      __builtin_amdgcn_sched_barrier(0);
       float rk[8], rv[8];
       tok_rows(A.L, x, kMerged, rk, rv);
       put_rows(rk, rv);
       __syncthreads();
       for (int g = 0; g < RPW && i0 + g < n; ++g) {
-        const int eg = lst[i0 + g];
+        const int eg = __builtin_amdgcn_readlane(e, g * GL);
         if (((eg >> 1) & 127) != my || (eg & 1)) continue;
         float xk[8], xv[8];
         load8f(&rows[g][0][part * 8], xk);
@@ -439,6 +534,10 @@ __global__ __launch_bounds__(kThreads) void k_state_bwd(StateBwdArgs A, UpdTable
       }
       __syncthreads();  // rows is rewritten by the next batch
     }
+    if (n == 0) {
+      fetch_first(u - 1);
+      fetch_grad(u - 1);
+    }
     if (j >= before_of(u) && j < before_of(u) + napp_of(u)) {  // the slot did not exist before
 #pragma unroll
       for (int e = 0; e < 8; ++e) acck[e] = accv[e] = sk[e] = sv[e] = 0.f;
@@ -448,7 +547,6 @@ __global__ __launch_bounds__(kThreads) void k_state_bwd(StateBwdArgs A, UpdTable
   if (j < L0) {
     Tok x;
     make_tok<D>(A, fetch_tok(R, j, part), part, w, bb, x);
-    float cdk[8], cdv[8];
     const int64_t o = (rowT + j) * D + part * 8;
     load8f(A.dk + o, cdk);
     load8f(A.dv + o, cdv);
@@ -488,13 +586,53 @@ __global__ __launch_bounds__(256) void k_state_bwd_ln(const float *part, int nwg
   if (tid == 0) out[f] = (wred[0] + wred[1]) + (wred[2] + wred[3]);
 }
 
+// dk16 / dv16 rows [t0, T) of every row: the tokens that the state does not
+// hold, whose gradient is the window's alone (blockIdx.y: 0 keys, 1 values).
+__global__ __launch_bounds__(256) void k_round_tail(StateBwdArgs A, int64_t t0, int64_t units_row) {
+  const int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x;  // unit of 8 features of (row, token)
+  if (i >= units_row * A.rows) return;
+  const int64_t o = (i / units_row) * A.T * A.L.head_dim + t0 * A.L.head_dim + (i % units_row) * 8;
+  float x[8];
+  load8f((blockIdx.y ? A.dv : A.dk) + o, x);
+  store8((blockIdx.y ? A.dv16 : A.dk16) + o, x);
+}
+
+// Workspace: the LayerNorm partials, then the grouped entries and their offsets.
+struct StateBwdLayout {
+  int64_t groups, ent, off, total;  // groups per row; byte offsets
+};
+StateBwdLayout state_bwd_layout(int64_t head_dim, int64_t rows, int64_t max_state_len, int64_t n_updates, int64_t C) {
+  const int64_t rpw = kThreads / (head_dim / 8);
+  StateBwdLayout l;
+  l.groups = (max_state_len + rpw - 1) / rpw;
+  l.ent = l.groups * rows * 2 * head_dim * 4;
+  l.off = l.ent + n_updates * rows * C * 4;
+  l.total = l.off + n_updates * rows * (l.groups + 1) * 4;
+  return l;
+}
+
 template <int D>
 hipError_t launch_d(const StateBwdArgs &a, const UpdTable &sched, float *part, hipStream_t s) {
   constexpr int RPW = kThreads / (D / 8);
-  const dim3 grid(unsigned((a.max_state_len + RPW - 1) / RPW), unsigned(a.rows));
-  hipLaunchKernelGGL((k_state_bwd<D>), grid, dim3(kThreads), size_t(a.L.chunk_len) * 4, s, a, sched, part);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
+  const StateBwdLayout l = state_bwd_layout(D, a.rows, a.max_state_len, a.n_updates, a.L.chunk_len);
+  const dim3 grid(unsigned(l.groups), unsigned(a.rows));
+  int32_t *ent = reinterpret_cast<int32_t *>(reinterpret_cast<unsigned char *>(part) + l.ent);
+  int32_t *off = reinterpret_cast<int32_t *>(reinterpret_cast<unsigned char *>(part) + l.off);
+  hipError_t e;
+  if (a.n_updates > 0) {
+    hipLaunchKernelGGL(k_route_sort<RPW>, dim3(unsigned(a.rows), unsigned(a.n_updates)), dim3(kThreads), 0, s,
+                       a.route_log, a.append_log, int(a.rows), int(a.L.chunk_len), int(l.groups), ent, off);
+    if ((e = hipGetLastError()) != hipSuccess) return e;
+  }
+  hipLaunchKernelGGL((k_state_bwd<D>), grid, dim3(kThreads), 0, s, a, sched, ent, off, part);
+  if ((e = hipGetLastError()) != hipSuccess) return e;
+  const int64_t t0 = a.L0 + a.n_updates * a.L.chunk_len;  // first token after the updates' (checked by the caller)
+  if (a.dk16 && t0 < a.T) {
+    const int64_t units_row = (a.T - t0) * (D / 8);
+    hipLaunchKernelGGL(k_round_tail, dim3(unsigned((units_row * a.rows + 255) / 256), 2), dim3(256), 0, s, a, t0,
+                       units_row);
+    if ((e = hipGetLastError()) != hipSuccess) return e;
+  }
   hipLaunchKernelGGL(k_state_bwd_ln, dim3(2 * D), dim3(256), 0, s, part, int(grid.x * grid.y), 2 * D,
                      a.d_ln);
   return hipGetLastError();
@@ -502,10 +640,9 @@ hipError_t launch_d(const StateBwdArgs &a, const UpdTable &sched, float *part, h
 
 }  // namespace
 
-int64_t state_bwd_workspace_bytes(int64_t head_dim, int64_t rows, int64_t max_state_len) {
-  const int64_t rpw = kThreads / (head_dim / 8);
-  const int64_t nwg = (max_state_len + rpw - 1) / rpw * rows;
-  return nwg * 2 * head_dim * 4;
+int64_t state_bwd_workspace_bytes(int64_t head_dim, int64_t rows, int64_t max_state_len, int64_t n_updates,
+                                  int64_t chunk_len) {
+  return state_bwd_layout(head_dim, rows, max_state_len, n_updates, chunk_len).total;
 }
 
 int64_t state_bwd_max_chunk() { return kMaxChunk; }

@@ -163,6 +163,7 @@ SIGNATURES = {
     "kvm_prefill_backward": (ctypes.c_int, [_P(KvmPrefillBwdDesc), _vp]),
     "kvm_state_backward_workspace_bytes": (_i64, [_P(KvmStateBwdDesc)]),
     "kvm_state_backward": (ctypes.c_int, [_P(KvmStateBwdDesc), _vp]),
+    "kvm_state_backward_rounded": (ctypes.c_int, [_P(KvmStateBwdDesc), _vp, _vp, _vp]),
     "kvm_prefix": (ctypes.c_int, [_P(KvmPrefixDesc), _vp]),
     "kvm_ring_write_dev": (ctypes.c_int, [_P(KvmLayer), _P(KvmSeq), _vp, _vp, _vp, _i64, _vp, _vp]),
     "kvm_decode_attention_dev": (ctypes.c_int, [_P(KvmLayer), _vp, _i64, _i64, _P(KvmState), _vp, ctypes.c_int32,

@@ -116,7 +116,12 @@ class KVMPrefillFunction(torch.autograd.Function):
         plan = res["plan"]
         dq, dk_w, dv_w, d_snap_k, d_snap_v, d_ts, d_tf = attention_backward(mixer, q, k, v, gate, res, dout)
         if plan.n_chunks > mixer.config.n_bswa_chunks:  # some query chunk read the memory state
-            dgate, d_ln = state_backward(mixer, k, v, gate, res, d_snap_k, d_snap_v, dk_w, dv_w)
+            rounded = None
+            if k.dtype == v.dtype == torch.bfloat16:  # rounded where the state's share is added
+                rounded = tuple(torch.empty(k.shape, device=k.device, dtype=torch.bfloat16) for _ in range(2))
+            dgate, d_ln = state_backward(mixer, k, v, gate, res, d_snap_k, d_snap_v, dk_w, dv_w, out=rounded)
+            if rounded is not None:
+                dk_w, dv_w = rounded
             glw, glb = d_ln[0], d_ln[1]
         else:
             dgate = torch.zeros(gate.shape, device=gate.device, dtype=torch.float32)
@@ -125,14 +130,16 @@ class KVMPrefillFunction(torch.autograd.Function):
                 glw.to(ln_w.dtype), glb.to(ln_b.dtype), d_ts.to(state_temp.dtype), d_tf.to(front_temp.dtype))
 
 
-def state_backward(mixer, k, v, gate, res, d_snap_k, d_snap_v, dk, dv):
+def state_backward(mixer, k, v, gate, res, d_snap_k, d_snap_v, dk, dv, out=None):
     """The memory state's share of the backward (``kvm_state_backward``).
 
     k, v: [B, Hkv, T, D] bf16 and gate [B, Hkv, T, 1] as the forward read
     them; ``res`` the forward's ``prefill_raw`` result (plan, route_log,
     append_log); d_snap_k / d_snap_v the snapshot-row gradients; dk / dv
     fp32 [B, Hkv, T, D] contiguous, to which the state's share is added in
-    place.  Returns dgate fp32 [B, Hkv, T] and the ln_s_k gradients [2, D].
+    place; with ``out``, two contiguous bf16 tensors of that shape, the sums
+    are rounded into them instead and dk / dv are left as they are.  Returns
+    dgate fp32 [B, Hkv, T] and the ln_s_k gradients [2, D].
     Reference: _live_state_dkdv_to_raw_grad_kernel, _reverse_route_scatter_grad_split_kernel,
     _initial_state_grad_kernel (model/kernels/kvm_triton_training_kernels.py:2093-2745)."""
     B, Hkv, T, D = k.shape
@@ -165,7 +172,14 @@ def state_backward(mixer, k, v, gate, res, d_snap_k, d_snap_v, dk, dv):
         raise ValueError("invalid state-backward descriptor: " + lib.kvm_last_error().decode())
     ws = torch.empty(max(nws, 16), device=dev, dtype=torch.uint8)
     d.workspace, d.workspace_bytes = ws.data_ptr(), nws
-    _lib.check(lib.kvm_state_backward(ctypes.byref(d), _lib.stream_handle(dev)), "kvm_state_backward")
+    if out is None:
+        _lib.check(lib.kvm_state_backward(ctypes.byref(d), _lib.stream_handle(dev)), "kvm_state_backward")
+    else:
+        for t in out:
+            if t.dtype != torch.bfloat16 or not t.is_contiguous() or tuple(t.shape) != (B, Hkv, T, D):
+                raise ValueError("out must be two contiguous bf16 [B, Hkv, T, D] tensors")
+        _lib.check(lib.kvm_state_backward_rounded(ctypes.byref(d), out[0].data_ptr(), out[1].data_ptr(),
+                                               _lib.stream_handle(dev)), "kvm_state_backward_rounded")
     del keep, ws
     return dgate, d_ln
 

@@ -260,3 +260,60 @@ def test_state_backward_matches_replay_autograd(B, Hkv, D, C, Tn, mode, gates):
         worst.append(f"{name} {rmax:.1e}/{rmean:.1e}")
         assert rmax <= 2e-3 and rmean <= 2e-4, f"d{name}: relative max {rmax:.3e}, mean {rmean:.3e}"
     T.log(f"[state-backward] relative max/mean error: {', '.join(worst)}")
+
+
+@pytest.mark.parametrize("B,Hkv,D,C,Tn,mode", [
+    (1, 2, 128, 200, 1300, "fixed"),      # up to 200 tokens of one update on one slot, ragged tail
+    (2, 1, 64, 128, 1111, "power_law"),
+    (1, 1, 128, 512, 1025, "fixed"),      # no update: the initial rows and the tail
+])
+def test_state_backward_skewed_routes_and_rounded_output(B, Hkv, D, C, Tn, mode):
+    """Routes that send most of an update to a few slots (more entries than a
+    wave holds at once) against the replay, and the bf16 output against the
+    rounded fp32 one, every token's row, bit for bit."""
+    if not torch.cuda.is_available():
+        pytest.skip("needs an MI355X")
+    from kvm_amd import training
+
+    T.log(f"[state-backward skew] B{B} Hkv{Hkv} D{D} C{C} T{Tn} {mode}")
+    cfg = T.mixer_config(Hkv, Hkv, D, C, rope=16, mode=mode, min_len=C, n_max=4, factor=8.0, expo=0.5, gate_initial=1)
+    gen = torch.Generator().manual_seed(6)
+    lnw, lnb = (1 + 0.1 * torch.randn(D, generator=gen)).bfloat16(), (0.1 * torch.randn(D, generator=gen)).bfloat16()
+    m = T.make_mixer(cfg, lnw, lnb, torch.ones(Hkv).bfloat16(), torch.ones(Hkv).bfloat16())
+    q, v = (torch.randn(B, Hkv, Tn, D, generator=gen).bfloat16().to(DEV) for _ in range(2))
+    k = (torch.randn(D, generator=gen) + 0.1 * torch.randn(B, Hkv, Tn, D, generator=gen)).bfloat16().to(DEV)
+    g = (1 + F.elu(torch.randn(B, Hkv, Tn, 1, generator=gen))).bfloat16().to(DEV)
+    with torch.no_grad():
+        res = m.prefill_raw(q, k, v, g, route_log=True)
+    plan, rows = res["plan"], B * Hkv
+    if plan.n_updates and mode == "fixed":
+        top = max(int(torch.bincount(r.long()).max()) for r in res["route_log"][:plan.n_updates].flatten(0, 1).cpu())
+        assert top > 64, "inputs did not skew the routes"
+    shape = (plan.n_updates + 1, rows, plan.max_state_len, D)
+    dsk, dsv = (torch.randn(shape, generator=gen).to(DEV) for _ in range(2))
+    win = [torch.randn(B, Hkv, Tn, D, generator=gen).to(DEV) for _ in range(2)]
+    dk, dv = (w.clone() for w in win)
+    dgate, d_ln = training.state_backward(m, k, v, g, res, dsk, dsv, dk, dv)
+    out = tuple(torch.full_like(k, float("nan")) for _ in range(2))
+    kept = [w.clone() for w in win]
+    dgate2, d_ln2 = training.state_backward(m, k, v, g, res, dsk, dsv, *kept, out=out)
+    assert torch.equal(out[0], dk.bfloat16()) and torch.equal(out[1], dv.bfloat16())
+    assert torch.equal(dgate, dgate2) and torch.equal(d_ln, d_ln2)
+    assert torch.equal(kept[0], win[0]) and torch.equal(kept[1], win[1])
+    lcfg = {"eps": 1e-5, "rope_partial_dim": 16, "gate_keys": 1, "gate_values": 1, "gate_appends": 0,
+            "gate_initial": 1}
+    leaves = [x.double().requires_grad_(True) for x in (k.reshape(rows, Tn, D), v.reshape(rows, Tn, D),
+                                                        g.reshape(rows, Tn), lnw.to(DEV), lnb.to(DEV))]
+    snaps = replay_snapshot_rows(*leaves, plan, res["route_log"], res["append_log"], lcfg)
+    total = sum((ka * dsk[s, :, :ka.size(1)]).sum() + (va * dsv[s, :, :va.size(1)]).sum()
+                for s, (ka, va) in enumerate(snaps))
+    ref = torch.autograd.grad(total, leaves)
+    got = ((dk - win[0]).view(rows, Tn, D), (dv - win[1]).view(rows, Tn, D), dgate.view(rows, Tn), d_ln[0], d_ln[1])
+    # fp32 sums: 1e-4 of the gradient.  The gate's is a dot product over D of
+    # key rows and their gradients that LayerNorm's scale invariance cancels
+    # for an initial row, so it also gets the rounding of its D terms,
+    # 2^-20 sqrt(D) of the key gradients' size.
+    slack = 2.0 ** -20 * D ** 0.5 * float(ref[0].norm())
+    for name, a, b in zip(["k", "v", "gate", "ln_w", "ln_b"], got, ref):
+        err, size = float((a - b).norm()), float(b.norm())
+        assert err <= 1e-4 * size + (slack if name == "gate" else 0), f"d{name}: error {err:.2e} of {size:.2e}"
