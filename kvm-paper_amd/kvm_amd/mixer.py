@@ -779,26 +779,33 @@ class SequenceMixer(nn.Module):
                       state_length_after_cycle(self.state_budget, self.chunk_len, self.n_bswa_chunks,
                                                int(T), plan.final_state_len, self.n_bswa_chunks * self.chunk_len))
         # The status word is read without stalling the GPU: the output
-        # projection is queued behind the prefill before the host waits for
-        # the word's copy.  A timed-out chain is repeated on the per-update
-        # kernels (bit-identical results), as prefill_raw does.
+        # projection and the decode cache's window copies are queued behind
+        # the prefill before the host waits for the word's copy, so the GPU
+        # works on while the host returns and queues what comes next.  A
+        # timed-out chain is repeated on the per-update kernels (bit-identical
+        # results), as prefill_raw does.
+        begin = self._bswa_begin_for_total_len(int(T))
+        if past_key_values is not None and plan.final_coverage != max(plan.initial_state_len, begin):
+            raise AssertionError("KVM prefill state progression drifted from cache bookkeeping.")
+
+        def finish(res):
+            y = self.c_proj(res["out"].view(B, T, -1))
+            if past_key_values is None:
+                return y, None
+            return y, self._cache_from_prefill(res, k, v, merge_gate, int(T), begin)
+
         res = self.prefill_raw(q, k, v, merge_gate, plan=plan, state_capacity=cap, check_status=False)
         status = self._status_pending(q.device)
-        y = self.c_proj(res["out"].view(B, T, -1))
+        y, cache = finish(res)
         bits = status()
         if bits & _lib.KVM_STATUS_CHAIN_TIMEOUT:
             warnings.warn("kvm_prefill: the persistent update chain timed out waiting for its row group "
                           "(another workload held compute units); repeating the prefill on the per-update "
                           "kernels", RuntimeWarning, stacklevel=2)
-            res = self.prefill_raw(q, k, v, merge_gate, plan=plan, state_capacity=cap, chain=False)
-            y = self.c_proj(res["out"].view(B, T, -1))
+            y, cache = finish(self.prefill_raw(q, k, v, merge_gate, plan=plan, state_capacity=cap, chain=False))
         else:
             self._raise_status(bits)
-        if past_key_values is not None:
-            begin = self._bswa_begin_for_total_len(int(T))
-            if plan.final_coverage != max(plan.initial_state_len, begin):
-                raise AssertionError("KVM prefill state progression drifted from cache bookkeeping.")
-            cache = self._cache_from_prefill(res, k, v, merge_gate, int(T), begin)
+        if cache is not None:
             past_key_values.update(self.layer_idx, offset=int(T), states_dict={self._CACHE_TRITON_DECODE: cache})
         return y
 
