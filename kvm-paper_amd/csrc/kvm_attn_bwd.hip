@@ -31,7 +31,19 @@
 //   dq kernel:   S^T = K Q^T, dP^T = V dO^T, dq^T += K^T dS^T;
 //   dkdv kernel: S = Q K^T, dP = dO V^T, dv^T += dO^T P, dk^T += Q^T dS;
 // P and dS never leave registers.  Each 64-row block is consumed as two
-// 32-row halves (fewer live score registers).
+// 32-row halves (fewer live score registers).  A block that every query sees
+// whole takes a path without tests or branches, both halves in one straight
+// line: the scores of the second half issue before the output products of the
+// first, so a wave has independent matrix work under its exponentials (at two
+// waves per SIMD the kernels wait on their own chains, not on LDS, L2 or the
+// matrix units: 26 - 44 % matrix-busy, 46 % of the wave cycles of the window
+// kernel waiting before).  Measured at 32768 tokens x 32 heads of 128: dq 1297
+// -> 1165 us, window dk/dv 1604 -> 1247; 2 x 16 (4 kv) heads of 64, 4099 tokens: dq 110
+// -> 79, window 45 -> 33, snapshots 87 -> 76.  32 keys per dk/dv wave, half
+// the LDS reads, were slower (2332 us: one wave per SIMD; 45 -> 64 us at
+// D = 64).
+
+#include <type_traits>
 
 #include "kvm_attn_tile.hpp"
 #include "kvm_device.hpp"
@@ -60,6 +72,42 @@ __device__ __forceinline__ int xcd_logical(int bid, int N) {
   const int x = bid % kXcds, jx = bid / kXcds;
   const int q8 = N / kXcds, r8 = N % kXcds;
   return x * q8 + min(x, r8) + jx;
+}
+
+// Order of a fully visible 64-query block in the dk/dv kernel at D = 128: the
+// first fragments ahead, then one MFMA at a time with the LDS reads of later
+// ones behind it, the weights of a half (VALU) under the scores and the output
+// products of the other.  Without it the compiler keeps too few LDS reads in
+// flight for two waves per SIMD (32768 tokens x 32 heads: window 1266 -> 1247
+// us, snapshots 852 -> 833).  At D = 64, with 3 or 4 waves per SIMD, it gains
+// nothing (33.2 -> 34.1, 75.6 -> 77.2 us), nor does the raised wave priority
+// of the output products there (75.6 -> 81.2), worth 14 % of the window kernel
+// at D = 128.
+__device__ __forceinline__ void interleave_block() {
+  constexpr int kMfma = 0x8, kLdsRead = 0x100, kValu = 0x2, kHalf = 16;  // 16 MFMAs per half and product pair
+  __builtin_amdgcn_sched_group_barrier(kLdsRead, 8, 0);
+#pragma unroll
+  for (int i = 0; i < kHalf; ++i) {  // scores of half 0
+    __builtin_amdgcn_sched_group_barrier(kMfma, 1, 0);
+    __builtin_amdgcn_sched_group_barrier(kLdsRead, 1, 0);
+  }
+#pragma unroll
+  for (int i = 0; i < kHalf; ++i) {  // scores of half 1, weights of half 0
+    __builtin_amdgcn_sched_group_barrier(kMfma, 1, 0);
+    __builtin_amdgcn_sched_group_barrier(kLdsRead, 1, 0);
+    __builtin_amdgcn_sched_group_barrier(kValu, 6, 0);
+  }
+#pragma unroll
+  for (int i = 0; i < kHalf; ++i) {  // products of half 0, weights of half 1
+    __builtin_amdgcn_sched_group_barrier(kMfma, 1, 0);
+    __builtin_amdgcn_sched_group_barrier(kLdsRead, 2, 0);
+    __builtin_amdgcn_sched_group_barrier(kValu, 6, 0);
+  }
+#pragma unroll
+  for (int i = 0; i < kHalf; ++i) {  // products of half 1
+    __builtin_amdgcn_sched_group_barrier(kMfma, 1, 0);
+    __builtin_amdgcn_sched_group_barrier(kLdsRead, 2, 0);
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -184,10 +232,9 @@ void k_attn_bwd_dq(kvm_layer L, BwdArgs A, int qtiles, ChunkTable table, float *
         const int nvalid = min(BN, nkeys - j * BN);
         const bool masked = nvalid < BN || qrel < BN - 1;
         const unsigned char *kimg = lds + (j & 1) * BUF, *vimg = kimg + BLK;
-#pragma unroll
-        for (int hb = 0; hb < 2; ++hb) {
-          if (nvalid <= 32 * hb || qrel + 31 < 32 * hb) continue;  // wave-uniform: nothing visible
-          // One 16-key tile at a time: S^T and dP^T, then its dS^T pairs.
+        // dS^T of the 32 keys of step hb (scaled by tau / sqrt(D)), in the
+        // B-operand layout, one 16-key tile at a time.
+        auto scores = [&](int hb, auto mask, bf16x8 (&dsb)[2]) {
           uint32_t pk[2][2][2];  // [rt][k2][pair]
 #pragma unroll
           for (int k2 = 0; k2 < 2; ++k2) {
@@ -214,7 +261,7 @@ void k_attn_bwd_dq(kvm_layer L, BwdArgs A, int qtiles, ChunkTable table, float *
 #pragma unroll
               for (int i = 0; i < 4; ++i) {
                 const int key = kt * 16 + (lane >> 4) * 4 + i;
-                const bool vis = !masked || (key < nvalid && (!causal || key <= lim));
+                const bool vis = !mask.value || (key < nvalid && (!causal || key <= lim));
                 const float p = vis ? __builtin_amdgcn_exp2f(__builtin_fmaf(s[rt][i], sc, -lse[rt])) : 0.f;
                 const float ds = p * (dp[rt][i] - dl[rt]);
                 tacc += ds * s[rt][i];
@@ -224,18 +271,35 @@ void k_attn_bwd_dq(kvm_layer L, BwdArgs A, int qtiles, ChunkTable table, float *
               pk[rt][k2][1] = pack_bf16x2(d[2], d[3]);
             }
           }
-          // dS^T (scaled by tau / sqrt(D)) in the B-operand layout of step hb.
-          bf16x8 dsb[2];
 #pragma unroll
           for (int rt = 0; rt < 2; ++rt)
             dsb[rt] = as_bf16x8(make_uint4(pk[rt][0][0], pk[rt][0][1], pk[rt][1][0], pk[rt][1][1]));
-          // dq^T += K^T dS^T over the 32 keys of step hb.
+        };
+        // dq^T += K^T dS^T over the 32 keys of step hb.
+        auto outer = [&](int hb, const bf16x8 (&dsb)[2]) {
+          if constexpr (D == 128) __builtin_amdgcn_s_setprio(1);
 #pragma unroll
           for (int dt = 0; dt < DT; ++dt) {
             const bf16x8 kt_f = tr_frag(kimg, lo, hb, dt);
 #pragma unroll
             for (int rt = 0; rt < 2; ++rt)
               dq[rt][dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kt_f, dsb[rt], dq[rt][dt], 0, 0, 0);
+          }
+          if constexpr (D == 128) __builtin_amdgcn_s_setprio(0);
+        };
+        if (!masked) {
+          bf16x8 ds0[2], ds1[2];
+          scores(0, std::false_type{}, ds0);
+          scores(1, std::false_type{}, ds1);
+          outer(0, ds0);
+          outer(1, ds1);
+        } else {
+#pragma unroll
+          for (int hb = 0; hb < 2; ++hb) {
+            if (nvalid <= 32 * hb || qrel + 31 < 32 * hb) continue;  // wave-uniform: nothing visible
+            bf16x8 dsb[2];
+            scores(hb, std::true_type{}, dsb);
+            outer(hb, dsb);
           }
         }
       }
@@ -430,6 +494,20 @@ void k_attn_bwd_dkdv(kvm_layer L, BwdArgs A, int kblocks, ChunkTable table) {
   const uint32_t qo = lo.drow * qstride_b + lo.dcol, doo = lo.drow * dstride_b + lo.dcol;
   const int nqb = int((tq_hi - tq_lo + BN - 1) / BN);
   const int64_t kp = kr;  // the lane's key (column lane%16 of every C tile)
+  // Query t sees key p iff, in the window, p <= t < (p/C + n) C (the chunk of
+  // t starts its window at or before p), and in a snapshot always.  Kept as
+  // offsets from tq_lo: [vis0, vis1) of the lane's key (empty for a key past
+  // the range), [all0, all1) seen by every key of the wave, [any0, any1) by
+  // some.  Following the chunk of every query block instead took two 64-bit
+  // scalar divisions per block and wave.
+  const int64_t kw = kb0 + wave * 16;  // the wave's first key
+  auto seen_end = [&](int64_t key) {
+    return int(SNAP ? tq_hi - tq_lo : min(tq_hi, (key / C + n) * int64_t(C)) - tq_lo);
+  };
+  const int vis0 = SNAP ? 0 : wave * 16 + (lane & 15);
+  const uint32_t vis_n = kok ? uint32_t(max(seen_end(kp) - vis0, 0)) : 0u;  // number of queries that see the key
+  const int all0 = SNAP ? 0 : wave * 16 + 15, all1 = kw + 16 <= nkeys ? seen_end(kw) : 0;
+  const int any0 = SNAP ? 0 : wave * 16, any1 = kw < nkeys ? seen_end(min(kw + 15, int64_t(nkeys) - 1)) : 0;
 #pragma unroll 1
   for (int h = 0; h < grp; ++h) {
     const int hq = hk * grp + h;
@@ -465,81 +543,66 @@ void k_attn_bwd_dkdv(kvm_layer L, BwdArgs A, int kblocks, ChunkTable table) {
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       __syncthreads();
       if (j + 1 < nqb) issue(j + 1);
-      const int64_t t0 = tq_lo + int64_t(j) * BN;
-      const int nq = int(min(int64_t(BN), tq_hi - t0));
+      const int t0 = j * BN;  // the block's first query, from tq_lo
       const unsigned char *qimg = lds + (j & 1) * BUF, *dimg = qimg + BLK;
-      // Window start of the chunks the block's queries lie in: with C >= 64
-      // a 64-query block spans at most two chunks, c0 and c0 + 1 (first
-      // query of c0 + 1 at `bnd`); shorter chunks take the division per query.
-      const int64_t c0 = t0 / C, bnd = (c0 + 1) * C;
-      const int64_t wb0 = max(int64_t(0), (c0 - n + 1) * int64_t(C)), wb1 = max(int64_t(0), (c0 - n + 2) * int64_t(C));
-      const bool two_chunks = C >= BN;
       const float *lse_s = &stat[j & 1][0][0], *dl_s = &stat[j & 1][1][0];
-#pragma unroll
-      for (int hb = 0; hb < 2; ++hb) {
-        // wave-uniform: no valid query in the half, or (window) all of its
-        // queries before the wave's first key
-        if (nq <= 32 * hb) continue;
-        if (!SNAP && t0 + 32 * hb + 31 < kb0 + wave * 16) continue;
-        f32x4 s[2], dp[2];
-#pragma unroll
-        for (int q2 = 0; q2 < 2; ++q2) {
-          const int qt = 2 * hb + q2;
-          s[q2] = f32x4{0.f, 0.f, 0.f, 0.f};
-          dp[q2] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-          for (int ks = 0; ks < KS; ++ks) {
-            s[q2] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(row_frag(qimg, lo, qt, ks), kf[ks], s[q2], 0, 0, 0);
-            dp[q2] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(row_frag(dimg, lo, qt, ks), vf[ks], dp[q2], 0, 0, 0);
-          }
-        }
-        // P and dS (scaled by tau / sqrt(D)) in the B-operand layout of step hb:
-        // lane holds queries qt*16 + 4*(lane/16) + i of key lane%16.
-        // Wave-uniform: every (query, key) pair of the step is visible (all 32
-        // queries valid, the wave's 16 keys valid and, in the window, at or
-        // before the first query and at or after the last query's window
-        // start), so no per-pair test is needed.
-        const int64_t kw = kb0 + wave * 16;
-        bool all_vis = 32 * hb + 32 <= nq && kw + 16 <= nkeys;
-        if (!SNAP) {
-          const int64_t qa = t0 + 32 * hb, qz = qa + 31;
-          all_vis = all_vis && kw + 15 <= qa && max(int64_t(0), (qz / C - n + 1) * int64_t(C)) <= kw;
-        }
+      // P and dS (scaled by tau / sqrt(D)) of the 32 queries of step hb in the
+      // B-operand layout: lane holds queries qt*16 + 4*(lane/16) + i of key lane%16.
+      auto scores = [&](int hb, auto mask, bf16x8 &pb, bf16x8 &db) {
         uint32_t pp[2][2], pd[2][2];
 #pragma unroll
         for (int q2 = 0; q2 < 2; ++q2) {
-          const int qr = (2 * hb + q2) * 16 + (lane >> 4) * 4;  // block-relative query of i = 0
+          const int qt = 2 * hb + q2;
+          f32x4 s = f32x4{0.f, 0.f, 0.f, 0.f}, dp = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+          for (int ks = 0; ks < KS; ++ks) {
+            s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(row_frag(qimg, lo, qt, ks), kf[ks], s, 0, 0, 0);
+            dp = __builtin_amdgcn_mfma_f32_16x16x32_bf16(row_frag(dimg, lo, qt, ks), vf[ks], dp, 0, 0, 0);
+          }
+          const int qr = qt * 16 + (lane >> 4) * 4;  // block-relative query of i = 0
           const float4 l4 = *reinterpret_cast<const float4 *>(lse_s + qr);
           const float4 d4 = *reinterpret_cast<const float4 *>(dl_s + qr);
           const float lv[4] = {l4.x, l4.y, l4.z, l4.w}, dv4[4] = {d4.x, d4.y, d4.z, d4.w};
           float p[4], d[4];
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
-            bool vis = true;
-            if (!all_vis) {
-              const int64_t t = t0 + qr + i;
-              vis = qr + i < nq && kp < nkeys;
-              if (!SNAP) {
-                const int64_t wbt =
-                    two_chunks ? (t < bnd ? wb0 : wb1) : max(int64_t(0), (t / C - n + 1) * int64_t(C));
-                vis = vis && kp <= t && wbt <= kp;
-              }
-            }
-            p[i] = vis ? __builtin_amdgcn_exp2f(__builtin_fmaf(s[q2][i], sc, -lv[i])) : 0.f;
-            d[i] = p[i] * (dp[q2][i] - dv4[i]) * dsc;
+            const bool vis = !mask.value || uint32_t(t0 + qr + i - vis0) < vis_n;
+            p[i] = vis ? __builtin_amdgcn_exp2f(__builtin_fmaf(s[i], sc, -lv[i])) : 0.f;
+            d[i] = p[i] * (dp[i] - dv4[i]) * dsc;
           }
           pp[q2][0] = pack_bf16x2(p[0], p[1]);
           pp[q2][1] = pack_bf16x2(p[2], p[3]);
           pd[q2][0] = pack_bf16x2(d[0], d[1]);
           pd[q2][1] = pack_bf16x2(d[2], d[3]);
         }
-        const bf16x8 pb = as_bf16x8(make_uint4(pp[0][0], pp[0][1], pp[1][0], pp[1][1]));
-        const bf16x8 db = as_bf16x8(make_uint4(pd[0][0], pd[0][1], pd[1][0], pd[1][1]));
-        // dv^T += dO^T P, dk^T += Q^T dS over the 32 queries of step hb.
+        pb = as_bf16x8(make_uint4(pp[0][0], pp[0][1], pp[1][0], pp[1][1]));
+        db = as_bf16x8(make_uint4(pd[0][0], pd[0][1], pd[1][0], pd[1][1]));
+      };
+      // dv^T += dO^T P, dk^T += Q^T dS over the 32 queries of step hb.
+      auto outer = [&](int hb, const bf16x8 &pb, const bf16x8 &db) {
+        if constexpr (D == 128) __builtin_amdgcn_s_setprio(1);
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt) {
           dv[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(tr_frag(dimg, lo, hb, dt), pb, dv[dt], 0, 0, 0);
           dk[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(tr_frag(qimg, lo, hb, dt), db, dk[dt], 0, 0, 0);
+        }
+        if constexpr (D == 128) __builtin_amdgcn_s_setprio(0);
+      };
+      if (t0 >= all0 && t0 + BN <= all1) {  // wave-uniform: every pair of the block is visible
+        bf16x8 p0, d0, p1, d1;
+        scores(0, std::false_type{}, p0, d0);
+        scores(1, std::false_type{}, p1, d1);
+        outer(0, p0, d0);
+        outer(1, p1, d1);
+        if constexpr (D == 128) interleave_block();
+      } else {
+#pragma unroll
+        for (int hb = 0; hb < 2; ++hb) {
+          // wave-uniform: no query of the half sees a key of the wave
+          if (t0 + 32 * hb + 31 < any0 || t0 + 32 * hb >= any1) continue;
+          bf16x8 pb, db;
+          scores(hb, std::true_type{}, pb, db);
+          outer(hb, pb, db);
         }
       }
     }

@@ -317,3 +317,10 @@ def test_state_backward_skewed_routes_and_rounded_output(B, Hkv, D, C, Tn, mode)
     for name, a, b in zip(["k", "v", "gate", "ln_w", "ln_b"], got, ref):
         err, size = float((a - b).norm()), float(b.norm())
         assert err <= 1e-4 * size + (slack if name == "gate" else 0), f"d{name}: error {err:.2e} of {size:.2e}"
+
+
+@pytest.mark.parametrize("D,C,Tn", [(128, 32, 229), (64, 48, 331), (128, 80, 405), (128, 192, 705)])
+def test_backward_chunk_edges_inside_query_blocks(D, C, Tn):
+    """Window ends that fall inside a 64-query block and inside a wave's 32 queries, ragged
+    lengths, whole and masked blocks in one pass; the bounds are those of the test above."""
+    test_backward_matches_fp32_autograd(1, 4, 2, D, C, Tn, "fixed", 1.0, (1, 1, 0, 0), {})
