@@ -38,7 +38,7 @@
 // waves per SIMD the kernels wait on their own chains, not on LDS, L2 or the
 // matrix units: 26 - 44 % matrix-busy, 46 % of the wave cycles of the window
 // kernel waiting before).  Measured at 32768 tokens x 32 heads of 128: dq 1297
-// -> 1165 us, window dk/dv 1604 -> 1247; 2 x 16 (4 kv) heads of 64, 4099 tokens: dq 110
+// -> 1165 us, window dk/dv 1604 -> 1206, snapshots 779 -> 830; 2 x 16 (4 kv) heads of 64, 4099 tokens: dq 110
 // -> 79, window 45 -> 33, snapshots 87 -> 76.  32 keys per dk/dv wave, half
 // the LDS reads, were slower (2332 us: one wave per SIMD; 45 -> 64 us at
 // D = 64).
@@ -74,37 +74,20 @@ __device__ __forceinline__ int xcd_logical(int bid, int N) {
   return x * q8 + min(x, r8) + jx;
 }
 
-// Order of a fully visible 64-query block in the dk/dv kernel at D = 128: the
-// first fragments ahead, then one MFMA at a time with the LDS reads of later
-// ones behind it, the weights of a half (VALU) under the scores and the output
-// products of the other.  Without it the compiler keeps too few LDS reads in
-// flight for two waves per SIMD (32768 tokens x 32 heads: window 1266 -> 1247
-// us, snapshots 852 -> 833).  At D = 64, with 3 or 4 waves per SIMD, it gains
-// nothing (33.2 -> 34.1, 75.6 -> 77.2 us), nor does the raised wave priority
-// of the output products there (75.6 -> 81.2), worth 14 % of the window kernel
-// at D = 128.
-__device__ __forceinline__ void interleave_block() {
-  constexpr int kMfma = 0x8, kLdsRead = 0x100, kValu = 0x2, kHalf = 16;  // 16 MFMAs per half and product pair
-  __builtin_amdgcn_sched_group_barrier(kLdsRead, 8, 0);
+// Order of the output products of a wholly visible block in the dk/dv kernel
+// at D = 128 (32 MFMAs, two transposing LDS reads each): sixteen reads ahead,
+// then one MFMA and the reads of a later one at a time.  Left to itself the
+// compiler keeps too few LDS reads in flight for two waves per SIMD.  The
+// products also run at a raised wave priority, so that the other wave's
+// exponentials fill their gaps and not the other way round.  32768 tokens x 32
+// heads: window 1464 us with neither, 1339 with the priority, 1206 with both;
+// snapshots 942 / 876 / 830.  At D = 64, with four waves per SIMD, neither
+// gains (priority: snapshots 76 -> 81 us; grouped reads: 33 -> 34, 76 -> 77).
+__device__ __forceinline__ void interleave_products() {
+  constexpr int kMfma = 0x8, kLdsRead = 0x100;
+  __builtin_amdgcn_sched_group_barrier(kLdsRead, 16, 0);
 #pragma unroll
-  for (int i = 0; i < kHalf; ++i) {  // scores of half 0
-    __builtin_amdgcn_sched_group_barrier(kMfma, 1, 0);
-    __builtin_amdgcn_sched_group_barrier(kLdsRead, 1, 0);
-  }
-#pragma unroll
-  for (int i = 0; i < kHalf; ++i) {  // scores of half 1, weights of half 0
-    __builtin_amdgcn_sched_group_barrier(kMfma, 1, 0);
-    __builtin_amdgcn_sched_group_barrier(kLdsRead, 1, 0);
-    __builtin_amdgcn_sched_group_barrier(kValu, 6, 0);
-  }
-#pragma unroll
-  for (int i = 0; i < kHalf; ++i) {  // products of half 0, weights of half 1
-    __builtin_amdgcn_sched_group_barrier(kMfma, 1, 0);
-    __builtin_amdgcn_sched_group_barrier(kLdsRead, 2, 0);
-    __builtin_amdgcn_sched_group_barrier(kValu, 6, 0);
-  }
-#pragma unroll
-  for (int i = 0; i < kHalf; ++i) {  // products of half 1
+  for (int i = 0; i < 32; ++i) {
     __builtin_amdgcn_sched_group_barrier(kMfma, 1, 0);
     __builtin_amdgcn_sched_group_barrier(kLdsRead, 2, 0);
   }
@@ -580,21 +563,23 @@ void k_attn_bwd_dkdv(kvm_layer L, BwdArgs A, int kblocks, ChunkTable table) {
       };
       // dv^T += dO^T P, dk^T += Q^T dS over the 32 queries of step hb.
       auto outer = [&](int hb, const bf16x8 &pb, const bf16x8 &db) {
-        if constexpr (D == 128) __builtin_amdgcn_s_setprio(1);
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt) {
           dv[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(tr_frag(dimg, lo, hb, dt), pb, dv[dt], 0, 0, 0);
           dk[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(tr_frag(qimg, lo, hb, dt), db, dk[dt], 0, 0, 0);
         }
-        if constexpr (D == 128) __builtin_amdgcn_s_setprio(0);
       };
       if (t0 >= all0 && t0 + BN <= all1) {  // wave-uniform: every pair of the block is visible
         bf16x8 p0, d0, p1, d1;
         scores(0, std::false_type{}, p0, d0);
         scores(1, std::false_type{}, p1, d1);
+        if constexpr (D == 128) __builtin_amdgcn_s_setprio(1);
         outer(0, p0, d0);
         outer(1, p1, d1);
-        if constexpr (D == 128) interleave_block();
+        if constexpr (D == 128) {
+          interleave_products();
+          __builtin_amdgcn_s_setprio(0);
+        }
       } else {
 #pragma unroll
         for (int hb = 0; hb < 2; ++hb) {
