@@ -443,10 +443,7 @@ int kvm_ring_write(const kvm_layer *layer, const kvm_seq *src, void *ring_k,
                    int64_t pos, void *stream);
 
 /* Scratch of kvm_decode_attention for a window of up to max_rows
- * (state + ring) key rows: the partials of 256-row segments.  With a
- * workspace of up to four times the bytes for the cache's capacity
- * (st->capacity + ring_cap rows), calls of few workgroups use segments of 128
- * or 64 rows, which are faster there and differ in summation order only. */
+ * (state + ring) key rows. */
 int64_t kvm_decode_workspace_bytes(const kvm_layer *layer, int64_t max_rows);
 
 /* Single-token attention over active_state_len memory slots and recent_len
@@ -491,8 +488,7 @@ int kvm_decode_step(const kvm_layer *layer, const void *q, int64_t q_sb, int64_t
  * kvm_decode_attention (model/kvm_triton_mixer.py:717-757, whose counters are
  * host values); the attention's grid covers st->capacity + ring_cap rows
  * (workspace: kvm_decode_workspace_bytes of that many rows), and its result
- * is bit-identical to kvm_decode_attention's for the same counters and
- * workspace size. */
+ * is bit-identical to kvm_decode_attention's for the same counters. */
 int kvm_ring_write_dev(const kvm_layer *layer, const kvm_seq *src, void *ring_k,
                        void *ring_v, void *ring_gate, int64_t ring_cap,
                        const int32_t *ctl, void *stream);

@@ -593,7 +593,7 @@ int kvm_decode_attention_dev(const kvm_layer *layer, const void *q, int64_t q_sb
     return fail(KVM_ESPACE, "decode workspace of %lld bytes is smaller than %lld",
                 (long long)workspace_bytes, (long long)need);
   KVM_HIP(kvm::launch_decode(*layer, q, q_sb, q_sh, *st, 0, ring_k, ring_v, ring_cap, 0, 0, out, o_sb, o_sh,
-                             workspace, workspace_bytes, as_stream(stream), ctl, int(pending), max_rows),
+                             workspace, as_stream(stream), ctl, int(pending), max_rows),
           "kvm_decode_attention_dev");
   return KVM_OK;
 }
@@ -614,7 +614,8 @@ int kvm_decode_attention_noalloc(const kvm_layer *layer, const void *q, int64_t 
   void *scratch = nullptr;
   KVM_HIP(kvm::decode_scratch(&scratch), "decode scratch address");
   return kvm_decode_attention(layer, q, q_sb, q_sh, st, active_state_len, ring_k, ring_v,
-                              ring_cap, ring_start, recent_len, out, o_sb, o_sh, scratch, need, stream);
+                              ring_cap, ring_start, recent_len, out, o_sb, o_sh, scratch,
+                              int64_t(KVM_DECODE_SCRATCH_BYTES), stream);
 }
 
 int kvm_decode_attention(const kvm_layer *layer, const void *q, int64_t q_sb,
@@ -643,7 +644,7 @@ int kvm_decode_attention(const kvm_layer *layer, const void *q, int64_t q_sb,
                 (long long)workspace_bytes, (long long)need);
   KVM_HIP(kvm::launch_decode(*layer, q, q_sb, q_sh, *st, active_state_len, ring_k,
                              ring_v, ring_cap, ring_start, recent_len, out, o_sb,
-                             o_sh, workspace, workspace_bytes, as_stream(stream)),
+                             o_sh, workspace, as_stream(stream)),
           "kvm_decode_attention");
   return KVM_OK;
 }
@@ -674,7 +675,7 @@ int kvm_decode_step(const kvm_layer *layer, const void *q, int64_t q_sb, int64_t
                 (long long)workspace_bytes, (long long)need);
   KVM_HIP(kvm::launch_decode(*layer, q, q_sb, q_sh, *st, active_state_len, ring_k, ring_v,
                              ring_cap, ring_start, recent_len, out, o_sb, o_sh, workspace,
-                             workspace_bytes, as_stream(stream), nullptr, 0, 0, src, ring_gate),
+                             as_stream(stream), nullptr, 0, 0, src, ring_gate),
           "kvm_decode_step");
   return KVM_OK;
 }

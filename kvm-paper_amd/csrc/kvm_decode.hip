@@ -6,15 +6,18 @@
 // (one program per (batch, q_head), serial scan).
 //
 // Here the key rows [memory slots ; window ring rows] of every
-// (batch, kv_head) are split into segments of 256 rows (128 or 64 where that
-// leaves compute units idle: decode_rows_per_wave).  A workgroup (4
+// (batch, kv_head) are split into segments of 256 rows.  A workgroup (4
 // waves) owns one segment of one kv row and serves every query head of that
 // kv head it is launched for (the GQA group shares each K/V read).  A wave
-// reads 64 (32, 16) rows with D/8 lanes per row, i.e. 4 (D=128) or 8 (D=64) whole
+// reads 64 rows with D/8 lanes per row, i.e. 4 (D=128) or 8 (D=64) whole
 // rows per 16-byte-per-lane load: each load instruction covers 1 KiB of
 // contiguous HBM.  Scores, the wave softmax and the PV accumulation are in
 // fp32; the 4 waves merge (max, sum, acc) through LDS, and a second kernel
-// merges the segments in a fixed order (deterministic split-K).
+// merges the segments in a fixed order (deterministic split-K).  The split
+// depends on the live rows alone, so a sequence's result has the same bits
+// whatever batch, cache capacity or workspace it is computed with (segments of
+// 64 rows for calls of few workgroups, 1.5 us faster at 4 x 6 heads of 768
+// rows, added in another order and needed a workspace four times as large).
 
 #include <mutex>
 
@@ -25,7 +28,9 @@
 namespace kvm {
 namespace {
 
+constexpr int kRowsPerWave = 64;
 constexpr int kWaves = 4;
+constexpr int kSegRows = kRowsPerWave * kWaves;
 constexpr float kLog2e = 1.4426950408889634f;
 
 // Non-temporal 16-byte load: every K/V row is read once per step, and the
@@ -37,8 +42,7 @@ __device__ __forceinline__ uint4 ld_stream16(const uint16_t *p) {
   return make_uint4(x[0], x[1], x[2], x[3]);
 }
 
-// RW: key rows per wave (64, 32 or 16).
-template <int D, int GQ, int RW>
+template <int D, int GQ>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(GQ == 1 ? 3 : 2))) void k_decode_partial(
     kvm_layer L, const uint16_t *__restrict__ q, int64_t q_sb, int64_t q_sh,
     const uint16_t *__restrict__ sk, const uint16_t *__restrict__ sv,
@@ -49,8 +53,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(GQ == 1 ? 3
     uint16_t *ring_k_out, uint16_t *ring_v_out, uint16_t *ring_g_out) {
   constexpr int G = D / 8;             // lanes per key row
   constexpr int RPS = 64 / G;          // rows per wave step
-  constexpr int STEPS = RW / RPS;
-  constexpr int kSegRows = RW * kWaves;
+  constexpr int STEPS = kRowsPerWave / RPS;
   __shared__ float sm_m[kWaves][GQ], sm_l[kWaves][GQ];
   __shared__ float sm_acc[kWaves][GQ][D];
 
@@ -78,7 +81,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(GQ == 1 ? 3
     tf[j] = static_cast<const float *>(L.front_temp)[hq0 + j];
   }
 
-  const int r0 = seg * kSegRows + wave * RW;
+  const int r0 = seg * kSegRows + wave * kRowsPerWave;
   const uint16_t *skrow = sk + int64_t(row) * cap * D;
   const uint16_t *svrow = sv + int64_t(row) * cap * D;
   const uint16_t *rkrow = rk + int64_t(row) * ring_cap * D;
@@ -97,6 +100,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(GQ == 1 ? 3
     gate_val = *(static_cast<const uint16_t *>(fresh.gate) + b * fresh.g_sb + hk * fresh.g_sh);
 
   // Issue every K and V load of the wave first (2 x STEPS x 16 B per lane).
+  // A row is a memory slot, the step's token or a row of the ring, which wraps
+  // at most once (0 <= ring_start < ring_cap): a 64-bit remainder per row took
+  // the launch pair of 4 x 6 heads of 768 rows from 8.8 to 10.6 us.
   uint4 kraw[STEPS], vraw[STEPS];
 #pragma unroll
   for (int s = 0; s < STEPS; ++s) {
@@ -104,23 +110,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(GQ == 1 ? 3
     kraw[s] = make_uint4(0, 0, 0, 0);
     vraw[s] = make_uint4(0, 0, 0, 0);
     if (r < total) {
-      int64_t o;
-      const uint16_t *kb, *vb;
-      if (r < active) {
-        o = int64_t(r) * D;
-        kb = skrow;
-        vb = svrow;
-      } else if (from_fresh && r == fresh_row) {
-        o = 0;
-        kb = fkrow;
-        vb = fvrow;
-      } else {
-        o = ((ring_start + (r - active)) % ring_cap) * D;
-        kb = rkrow;
-        vb = rvrow;
-      }
-      kraw[s] = ld_stream16(kb + o + part * 8);
-      vraw[s] = ld_stream16(vb + o + part * 8);
+      const uint32_t i = uint32_t(ring_start) + uint32_t(r - active);
+      const bool slot = r < active, token = from_fresh && r == fresh_row;
+      const int64_t o = int64_t(slot ? uint32_t(r) : i >= uint32_t(ring_cap) ? i - uint32_t(ring_cap) : i) * D;
+      kraw[s] = ld_stream16((token ? fkrow : (slot ? skrow : rkrow) + o) + part * 8);
+      vraw[s] = ld_stream16((token ? fvrow : (slot ? svrow : rvrow) + o) + part * 8);
     }
   }
 
@@ -266,7 +260,7 @@ __global__ __launch_bounds__(D) void k_decode_combine(
   out[b * o_sb + h * o_sh + d] = uint16_t(f2bf(a / l));
 }
 
-template <int D, int GQ, int RW>
+template <int D, int GQ>
 hipError_t launch_partial(const kvm_layer &L, const void *q, int64_t q_sb,
                           int64_t q_sh, const kvm_state &st, int64_t active,
                           const void *ring_k, const void *ring_v,
@@ -277,7 +271,7 @@ hipError_t launch_partial(const kvm_layer &L, const void *q, int64_t q_sb,
   const int group = int(L.q_heads / L.kv_heads);
   dim3 grid(unsigned(nseg), unsigned(L.batch * L.kv_heads),
             unsigned(group / GQ));
-  hipLaunchKernelGGL((k_decode_partial<D, GQ, RW>), grid, dim3(256), 0, stream, L,
+  hipLaunchKernelGGL((k_decode_partial<D, GQ>), grid, dim3(256), 0, stream, L,
                      static_cast<const uint16_t *>(q), q_sb, q_sh,
                      static_cast<const uint16_t *>(st.s_k_attn),
                      static_cast<const uint16_t *>(st.s_v_attn), st.capacity,
@@ -288,7 +282,7 @@ hipError_t launch_partial(const kvm_layer &L, const void *q, int64_t q_sb,
   return hipGetLastError();
 }
 
-template <int D, int RW>
+template <int D>
 hipError_t launch_partial_d(const kvm_layer &L, const void *q, int64_t q_sb,
                             int64_t q_sh, const kvm_state &st, int64_t active,
                             const void *ring_k, const void *ring_v,
@@ -297,17 +291,18 @@ hipError_t launch_partial_d(const kvm_layer &L, const void *q, int64_t q_sb,
                             float *pml, const int32_t *ctl, int pending, const kvm_seq &fresh,
                             uint16_t *rkw, uint16_t *rvw, uint16_t *rgw, hipStream_t stream) {
   // Query heads per workgroup: as many as share the key rows (4, 2, 1), but
-  // fewer where that would leave compute units idle (two workgroups each):
-  // one head of 64 key rows after another is a chain, and the rows read again
-  // come from the caches.  B 1, 32 heads over 8, 768 rows of 128: 9.3 us with
-  // four heads per workgroup, 7.7 with one.  Each head's arithmetic is the same.
+  // fewer while that leaves compute units without a workgroup: one head of 64
+  // key rows after another is a chain, and the rows read again come from the
+  // caches.  32 heads over 8, 768 rows of 128, us of the launch pair with 4 /
+  // 2 / 1 heads: B 1 13.8 / 9.9 / 8.8, B 8 14.9 / 14.3 / 14.9, B 16 21.7 /
+  // 22.2 / 28.0.  Each head's arithmetic is the same.
   const int64_t group = L.q_heads / L.kv_heads, wgs = L.batch * L.kv_heads * nseg;
   int64_t gq = group % 4 == 0 ? 4 : group % 2 == 0 ? 2 : 1;
-  while (gq > 1 && wgs * (group / gq) < 512) gq /= 2;
+  while (gq > 1 && wgs * (group / gq) < 256) gq /= 2;
 #define KVM_PARTIAL(GQ)                                                      \
-  launch_partial<D, GQ, RW>(L, q, q_sb, q_sh, st, active, ring_k, ring_v,   \
-                            ring_cap, ring_start, recent_len, nseg, pacc,   \
-                            pml, ctl, pending, fresh, rkw, rvw, rgw, stream)
+  launch_partial<D, GQ>(L, q, q_sb, q_sh, st, active, ring_k, ring_v,       \
+                        ring_cap, ring_start, recent_len, nseg, pacc, pml, \
+                        ctl, pending, fresh, rkw, rvw, rgw, stream)
   if (gq == 4) return KVM_PARTIAL(4);
   if (gq == 2) return KVM_PARTIAL(2);
   return KVM_PARTIAL(1);
@@ -329,42 +324,11 @@ void launch_combine(const kvm_layer &L, int nseg, const float *pacc, const float
 
 }  // namespace
 
-namespace {
-int64_t segments(int64_t rows_total, int rw) { return (rows_total + rw * kWaves - 1) / (rw * kWaves); }
-int64_t partial_bytes(const kvm_layer &L, int64_t nseg) { return L.batch * L.q_heads * nseg * (L.head_dim + 2) * 4; }
-
-// Key rows per wave for a cache of `max_rows` rows (memory slots + window).
-// 64 fill the memory pipeline best where the launch has workgroups to spare
-// (B 64, 32 heads, 1536 rows: 233 us a step).  With few workgroups a step is
-// the latency of one wave's rows, and shorter segments win: D 128, 768 rows,
-// one launch pair, in us with 64 / 32 / 16 rows per wave:
-//   B 4, 6 heads (72 workgroups of 256 rows)     10.9 / 8.8 / 7.7
-//   B 8, 32 heads over 8 (192)                   16.5 / 14.4 / 13.2
-//   B 16, 32 heads over 8 (384)                  22.4 / 18.0 / 17.6
-//   B 8, 32 heads (768)                          17.8 / 15.3 / 15.1
-//   B 4, 32 heads of 64, 1536 rows (768)         12.5 / 11.7 / 13.2
-// At most 16 segments, which the combine kernel loads at once (32 cost it
-// 1.2 us more: B 1, 32 heads, 2048 rows 12.4 us with 16 rows per wave, 10.7
-// with 32), and only where
-// the caller's workspace holds their partials (kvm_decode_workspace_bytes
-// asks for those of 256-row segments, the least that a call needs).
-// The rule reads the cache's capacity, not the live rows, so that an eager
-// and a captured step on one workspace add in the same order.
-int decode_rows_per_wave(const kvm_layer &L, int64_t max_rows, int64_t workspace_bytes) {
-  const int64_t group = L.q_heads / L.kv_heads;
-  const int64_t gq = group % 4 == 0 ? 4 : group % 2 == 0 ? 2 : 1;
-  const int64_t wgs = L.batch * L.kv_heads * (group / gq) * segments(max_rows, 64);
-  const auto fits = [&](int rw) {
-    return segments(max_rows, rw) <= 16 && partial_bytes(L, segments(max_rows, rw)) <= workspace_bytes;
-  };
-  if (wgs <= 256 && fits(16)) return 16;
-  if (wgs <= 1024 && fits(32)) return 32;
-  return 64;
-}
-}  // namespace
+int64_t decode_segments(int64_t rows_total) { return (rows_total + kSegRows - 1) / kSegRows; }
 
 int64_t decode_workspace_bytes(const kvm_layer &L, int64_t max_rows) {
-  return partial_bytes(L, segments(max_rows < 1 ? 1 : max_rows, 64));
+  const int64_t nseg = decode_segments(max_rows < 1 ? 1 : max_rows);
+  return L.batch * L.q_heads * nseg * (L.head_dim + 2) * 4;
 }
 
 // ---------------------------------------------------------------------------
@@ -404,7 +368,7 @@ hipError_t launch_decode(const kvm_layer &L, const void *q, int64_t q_sb,
                          const void *ring_k, const void *ring_v,
                          int64_t ring_cap, int64_t ring_start,
                          int64_t recent_len, void *out, int64_t o_sb,
-                         int64_t o_sh, void *workspace, int64_t workspace_bytes, hipStream_t stream,
+                         int64_t o_sh, void *workspace, hipStream_t stream,
                          const int32_t *ctl, int pending, int64_t max_rows,
                          const kvm_seq *fresh, void *ring_gate) {
   // Host counters: segments for the rows present; device counters: for
@@ -417,20 +381,19 @@ hipError_t launch_decode(const kvm_layer &L, const void *q, int64_t q_sb,
   uint16_t *rk = static_cast<uint16_t *>(const_cast<void *>(ring_k));
   uint16_t *rv = static_cast<uint16_t *>(const_cast<void *>(ring_v));
   uint16_t *rg = static_cast<uint16_t *>(ring_gate);
-  const int rw = decode_rows_per_wave(L, st.capacity + ring_cap, workspace_bytes);
-  const int nseg = int(segments(ctl ? max_rows : active + recent_len, rw));
+  const int nseg = int(decode_segments(ctl ? max_rows : active + recent_len));
   const int64_t npid = L.batch * L.q_heads;
   float *pacc = static_cast<float *>(workspace);
   float *pml = pacc + npid * nseg * L.head_dim;
   hipError_t e;
-#define KVM_PARTIAL_D(D, RW)                                                                                    \
-  launch_partial_d<D, RW>(L, q, q_sb, q_sh, st, active, ring_k, ring_v, ring_cap, ring_start, recent_len, nseg, \
-                          pacc, pml, ctl, pending, fr, rk, rv, rg, stream)
   if (L.head_dim == 128)
-    e = rw == 64 ? KVM_PARTIAL_D(128, 64) : rw == 32 ? KVM_PARTIAL_D(128, 32) : KVM_PARTIAL_D(128, 16);
+    e = launch_partial_d<128>(L, q, q_sb, q_sh, st, active, ring_k, ring_v,
+                              ring_cap, ring_start, recent_len, nseg, pacc,
+                              pml, ctl, pending, fr, rk, rv, rg, stream);
   else
-    e = rw == 64 ? KVM_PARTIAL_D(64, 64) : rw == 32 ? KVM_PARTIAL_D(64, 32) : KVM_PARTIAL_D(64, 16);
-#undef KVM_PARTIAL_D
+    e = launch_partial_d<64>(L, q, q_sb, q_sh, st, active, ring_k, ring_v,
+                             ring_cap, ring_start, recent_len, nseg, pacc, pml,
+                             ctl, pending, fr, rk, rv, rg, stream);
   if (e != hipSuccess) return e;
   if (L.head_dim == 128)
     launch_combine<128>(L, nseg, pacc, pml, out, o_sb, o_sh, stream);

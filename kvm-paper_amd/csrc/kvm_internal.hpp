@@ -145,6 +145,7 @@ hipError_t launch_ring_write(const kvm_layer &L, const kvm_seq &src,
                              int64_t ring_cap, int64_t pos, hipStream_t stream,
                              const int32_t *ctl = nullptr);
 
+int64_t decode_segments(int64_t rows_total);
 // Address of this device's library-owned decode scratch
 // (KVM_DECODE_SCRATCH_BYTES, resolved once per device).
 hipError_t decode_scratch(void **ptr);
@@ -154,7 +155,7 @@ hipError_t launch_decode(const kvm_layer &L, const void *q, int64_t q_sb,
                          const void *ring_k, const void *ring_v,
                          int64_t ring_cap, int64_t ring_start,
                          int64_t recent_len, void *out, int64_t o_sb,
-                         int64_t o_sh, void *workspace, int64_t workspace_bytes, hipStream_t stream,
+                         int64_t o_sh, void *workspace, hipStream_t stream,
                          const int32_t *ctl = nullptr, int pending = 0, int64_t max_rows = 0,
                          const kvm_seq *fresh = nullptr, void *ring_gate = nullptr);
 hipError_t launch_decode_advance(int32_t *ctl, int64_t n, hipStream_t stream);

@@ -141,8 +141,6 @@ class KVMDecodeCache:
     def _alloc_decode_workspace(self) -> None:
         lib = _lib.load()
         n = int(lib.kvm_decode_workspace_bytes(self.layer.ref(), self.state_capacity + self.ring_capacity))
-        if n <= 4 << 20:  # a small call: room for segments of 64 rows instead of 256 (kvm_decode_workspace_bytes)
-            n *= 4
         self.decode_workspace = torch.empty(max(n, 256), device=self.device, dtype=torch.uint8)
 
     def state_struct(self) -> _lib.KvmState:
