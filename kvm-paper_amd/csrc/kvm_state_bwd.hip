@@ -33,8 +33,11 @@
 // one per lane group whatever slot they belong to (the per-token LayerNorm
 // and chain rule keep every lane busy); their rows and the slots' gradients
 // cross between lane groups through LDS, and each owner folds its tokens in
-// list (token) order.  Every state token is routed to exactly one slot, so
-// each token row of dk / dv / dgate has exactly one writer (no atomics).
+// list (token) order.  A state token is routed to one slot, or to none (its
+// scores are all NaN, as with a NaN or infinite merge gate: route -1), so each
+// token row of dk / dv / dgate has at most one writer (no atomics).  Where the
+// sums are rounded into another array, k_route_sort writes the rows of the
+// tokens without a slot and k_round_tail those past the last update.
 
 #include "kvm_device.hpp"
 #include "kvm_internal.hpp"
@@ -212,11 +215,14 @@ __device__ __forceinline__ void tok_backward(const StateBwdArgs &A, const Tok &x
 // placement 64 tokens at a time (ballots over the group index).  The state
 // kernel used to compact the routes in every wave, in both scans: 17 % of its
 // instructions.
+// With A.dk16 set, the tokens that no slot took (route < 0: in no group) get
+// their rounded rows here, their gradient being the window's alone; the
+// updates' chunks then follow each other from token L0 on (checked by the caller).
 template <int RPW>
-__global__ __launch_bounds__(kThreads) void k_route_sort(const int32_t *route, const int32_t *append, int rows, int C,
-                                                         int ngrp, int32_t *ent, int32_t *off) {
+__global__ __launch_bounds__(kThreads) void k_route_sort(StateBwdArgs A, int ngrp, int32_t *ent, int32_t *off) {
   __shared__ int fill[kSortGroups];
-  const int lane = threadIdx.x;
+  const int lane = threadIdx.x, rows = int(A.rows), C = int(A.L.chunk_len);
+  const int32_t *route = A.route_log, *append = A.append_log;
   const int64_t ur = int64_t(blockIdx.y) * rows + blockIdx.x;  // (update, row)
   route += ur * C;
   append += ur * C;
@@ -267,6 +273,21 @@ __global__ __launch_bounds__(kThreads) void k_route_sort(const int32_t *route, c
     }
   }
   if (lane == 0) off[ngrp] = base;
+  if (A.dk16) {
+    constexpr int GL = kThreads / RPW, D = GL * 8;
+    const int64_t tok0 = blockIdx.x * A.T + A.L0 + int64_t(blockIdx.y) * C;
+    for (int t0 = 0; t0 < C; t0 += kThreads) {
+      uint64_t left = __ballot(t0 + lane < C && route[min(t0 + lane, C - 1)] < 0);
+      for (; left; left &= left - 1) {
+        const int64_t o = (tok0 + t0 + __builtin_ctzll(left)) * D + lane % GL * 8;
+        if (lane < 2 * GL) {
+          float x[8];
+          load8f((lane < GL ? A.dk : A.dv) + o, x);
+          store8((lane < GL ? A.dk16 : A.dv16) + o, x);
+        }
+      }
+    }
+  }
 }
 
 // Bound by VALU issue (the tokens' LayerNorms and chain rule, the slots'
@@ -621,7 +642,7 @@ hipError_t launch_d(const StateBwdArgs &a, const UpdTable &sched, float *part, h
   hipError_t e;
   if (a.n_updates > 0) {
     hipLaunchKernelGGL(k_route_sort<RPW>, dim3(unsigned(a.rows), unsigned(a.n_updates)), dim3(kThreads), 0, s,
-                       a.route_log, a.append_log, int(a.rows), int(a.L.chunk_len), int(l.groups), ent, off);
+                       a, int(l.groups), ent, off);
     if ((e = hipGetLastError()) != hipSuccess) return e;
   }
   hipLaunchKernelGGL((k_state_bwd<D>), grid, dim3(kThreads), 0, s, a, sched, ent, off, part);

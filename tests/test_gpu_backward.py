@@ -324,3 +324,42 @@ def test_backward_chunk_edges_inside_query_blocks(D, C, Tn):
     """Window ends that fall inside a 64-query block and inside a wave's 32 queries, ragged
     lengths, whole and masked blocks in one pass; the bounds are those of the test above."""
     test_backward_matches_fp32_autograd(1, 4, 2, D, C, Tn, "fixed", 1.0, (1, 1, 0, 0), {})
+
+
+@pytest.mark.parametrize("B,Hkv,D,C,Tn", [(1, 2, 128, 200, 1300), (2, 1, 64, 128, 1111)])
+def test_state_backward_rounds_tokens_that_no_slot_took(B, Hkv, D, C, Tn):
+    """A token whose gate is NaN or infinite scores NaN against every slot and
+    is routed to none: its row of the bf16 output is its window gradient, as in
+    the fp32 form, and not what the memory held before."""
+    if not torch.cuda.is_available():
+        pytest.skip("needs an MI355X")
+    from kvm_amd import training
+
+    T.log(f"[state-backward unrouted] B{B} Hkv{Hkv} D{D} C{C} T{Tn}")
+    cfg = T.mixer_config(Hkv, Hkv, D, C, rope=16, mode="fixed", min_len=C)
+    gen = torch.Generator().manual_seed(9)
+    lnw, lnb = (1 + 0.1 * torch.randn(D, generator=gen)).bfloat16(), (0.1 * torch.randn(D, generator=gen)).bfloat16()
+    m = T.make_mixer(cfg, lnw, lnb, torch.ones(Hkv).bfloat16(), torch.ones(Hkv).bfloat16())
+    q, k, v = (torch.randn(B, Hkv, Tn, D, generator=gen).bfloat16().to(DEV) for _ in range(3))
+    g = (1 + F.elu(torch.randn(B, Hkv, Tn, 1, generator=gen))).bfloat16().to(DEV)
+    bad = {C: math.nan, C + 1: math.inf, 2 * C - 1: -math.inf, 2 * C + 64: math.nan}  # tokens of the first two updates
+    for t, x in bad.items():
+        g[:, :, t] = x
+    with torch.no_grad():
+        res = m.prefill_raw(q, k, v, g, route_log=True)
+    plan, rows = res["plan"], B * Hkv
+    assert plan.upd_token_begin[:2] == [C, 2 * C]
+    for t in bad:
+        assert bool((res["route_log"][t // C - 1].view(rows, C)[:, t % C] == -1).all()), f"token {t} was routed"
+    shape = (plan.n_updates + 1, rows, plan.max_state_len, D)
+    dsk, dsv = (torch.randn(shape, generator=gen).to(DEV) for _ in range(2))
+    win = [torch.randn(B, Hkv, Tn, D, generator=gen).to(DEV) for _ in range(2)]
+    dk, dv = (w.clone() for w in win)
+    dgate, _ = training.state_backward(m, k, v, g, res, dsk, dsv, dk, dv)
+    out = tuple(torch.full_like(k, float("nan")) for _ in range(2))
+    training.state_backward(m, k, v, g, res, dsk, dsv, *win, out=out)
+    for name, got, want in (("dk", out[0], dk), ("dv", out[1], dv)):
+        wrong = (got != want.bfloat16()).any(-1).nonzero().tolist()
+        assert not wrong, f"{name} rows (batch, head, token) {wrong[:8]}"
+    for t in bad:
+        assert torch.equal(dk[:, :, t], win[0][:, :, t]) and not bool(dgate[:, :, t].any())
