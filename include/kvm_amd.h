@@ -391,6 +391,15 @@ const char *kvm_last_error(void);
  * max_state_len set). */
 int64_t kvm_prefill_workspace_bytes(const kvm_prefill_desc *d);
 
+/* How a prefill of states up to max_state_len slots runs its updates on a GPU
+ * of compute_units compute units (0: the current device; otherwise host
+ * arithmetic, no GPU needed): shape = {workgroups per row and rows per launch
+ * of batches with appends, the same of batches without appends at state_len
+ * slots}.  {0, 0, 0, 0}: the per-update kernels; 0 in the last two: the
+ * kernel of batches with appends. */
+int kvm_chain_shape(const kvm_layer *layer, int64_t max_state_len, int64_t state_len,
+                    int64_t compute_units, int32_t *shape);
+
 /* Whole prefill: initial state from the first chunk, every block-boundary
  * update of the schedule, and the attention of every query chunk.
  * Replaces build_prefill_forward (model/kernels/kvm_triton_training_kernels.py:3386-3619)

@@ -340,6 +340,23 @@ int64_t kvm_decode_workspace_bytes(const kvm_layer *layer, int64_t max_rows) {
   return kvm::decode_workspace_bytes(*layer, max_rows);
 }
 
+int kvm_chain_shape(const kvm_layer *layer, int64_t max_state_len, int64_t state_len, int64_t compute_units,
+                    int32_t *shape) {
+  int rc = check_layer(layer);
+  if (rc != KVM_OK) return rc;
+  if (!shape || max_state_len < 1 || compute_units < 0)
+    return fail(KVM_EINVAL, "chain shape: arguments out of range");
+  kvm::ChainPlan p;
+  const bool ok = compute_units > 0
+                      ? kvm::chain_plan_on(compute_units, *layer, layer->chunk_len, max_state_len, &p)
+                      : kvm::chain_plan(*layer, layer->chunk_len, max_state_len, &p);
+  if (ok)
+    kvm::chain_shape(p, state_len, layer->chunk_len, shape);
+  else
+    std::fill(shape, shape + 4, 0);
+  return KVM_OK;
+}
+
 int64_t kvm_prefill_workspace_bytes(const kvm_prefill_desc *d) {
   if (!d || check_layer(&d->layer) != KVM_OK) return -1;
   if (d->max_state_len < 1 || d->snapshot_ring < 2) return -1;

@@ -1982,13 +1982,22 @@ __global__ __launch_bounds__(256) void k_fill_u32(unsigned *p, int64_t n, unsign
 
 }  // namespace
 
+namespace {
+// Rows of G members that one launch keeps resident: one group per XCD at a
+// time, so whole eights.  0 where the device does not hold eight groups.
+int rows_per_launch(int64_t limit, int G) { return int(limit / G / 8 * 8); }
+}  // namespace
+
 bool chain_plan(const kvm_layer &L, int64_t n_tok, int64_t max_slots, ChainPlan *p) {
-  // Every member of a group must be resident at once: at most one
-  // workgroup per compute unit of the current device.
   int dev = 0, cus = 0;
-  if (hipGetDevice(&dev) != hipSuccess ||
-      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
-    return false;
+  return hipGetDevice(&dev) == hipSuccess &&
+         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess &&
+         chain_plan_on(cus, L, n_tok, max_slots, p);
+}
+
+bool chain_plan_on(int64_t cus, const kvm_layer &L, int64_t n_tok, int64_t max_slots, ChainPlan *p) {
+  // Every member of a group must be resident at once: at most one
+  // workgroup per compute unit.
   const int64_t limit = std::min<int64_t>(kChainMaxWorkgroups, cus);
   const int64_t rows = L.batch * L.kv_heads;
   const int64_t groups = (rows + 7) / 8 * 8;
@@ -2003,7 +2012,7 @@ bool chain_plan(const kvm_layer &L, int64_t n_tok, int64_t max_slots, ChainPlan 
     if ((G == 16 && groups * 16 > limit) || (G == 4 && groups * 8 <= limit)) continue;
     const int64_t tpw = ((n_tok + G - 1) / G + 15) / 16 * 16;
     const int64_t own_cap = ((max_slots + 15) / 16 + G - 1) / G * 16;
-    if (tpw > kChainTok || limit / G < 8 || n_tok < 1 || max_slots > 32768) continue;
+    if (tpw > kChainTok || rows_per_launch(limit, G) == 0 || n_tok < 1 || max_slots > 32768) continue;
     const int64_t dyn = append_lds_bytes(int(n_tok), int(own_cap));
     if (dyn > kAppendDynLds) continue;
     p->fixed = false;
@@ -2036,25 +2045,29 @@ namespace {
 int fixed_group(const ChainPlan &p, int S, int64_t n_tok) {
   if (n_tok > kFixedMaxTok) return 0;
   const int nblk = (S + 15) / 16;
-  // Owned slots per member: up to 64 at G = 16, up to 128 below; at most kChainTok prep tokens.
+  // Owned slots per member: up to 64 at G = 16, up to 128 below; at most kChainTok prep tokens;
+  // and a launch that holds eight groups, which the plan has checked for its own G only.
   const auto fits = [&](int G) {
-    return (nblk + G - 1) / G * 16 <= (G == 16 ? 64 : kOwnMax) && (n_tok + G - 1) / G <= kChainTok;
+    return rows_per_launch(p.limit, G) > 0 && (nblk + G - 1) / G * 16 <= (G == 16 ? 64 : kOwnMax) && (n_tok + G - 1) / G <= kChainTok;
   };
   if (p.G == 16) return fits(16) ? 16 : 0;
   const double work = double(n_tok + S) * p.head_dim / 128;
-  const auto launches = [&](int G) { return double((p.rows + p.limit / G - 1) / (p.limit / G)); };
+  const auto launches = [&](int G) {
+    const int per = G == 1 ? p.limit : rows_per_launch(p.limit, G);
+    return double((p.rows + per - 1) / per);
+  };
   int best = 0;
   double least = 0;
-  const auto offer = [&](int G, bool ok, double us) {
-    if (ok && (best == 0 || us < least)) {
+  const auto offer = [&](int G, double us) {
+    if (best == 0 || us < least) {
       best = G;
       least = us;
     }
   };
   const int rmax = p.head_dim == 128 ? RowMax<128>::value : RowMax<64>::value;
-  offer(8, fits(8), launches(8) * (5.2 + 0.0075 * work));
-  offer(4, fits(4), launches(4) * (4.0 + 0.016 * work));
-  offer(1, S <= rmax && n_tok <= rmax, launches(1) * (1.5 + 0.058 * work));
+  if (fits(8)) offer(8, launches(8) * (5.2 + 0.0075 * work));
+  if (fits(4)) offer(4, launches(4) * (4.0 + 0.016 * work));
+  if (S <= rmax && n_tok <= rmax) offer(1, launches(1) * (1.5 + 0.058 * work));
   return best;
 }
 }  // namespace
@@ -2065,6 +2078,14 @@ bool chain_fixed_ok(const ChainPlan &p, const ChainList &list, int64_t n_tok) {
   for (int i = 0; i < list.count; ++i)
     if (list.n_append[i] != 0 || list.state_before[i] != S) return false;
   return fixed_group(p, S, n_tok) != 0;
+}
+
+void chain_shape(const ChainPlan &p, int64_t state_len, int64_t n_tok, int32_t *shape) {
+  const int G = state_len >= 1 && state_len <= 0x7fff ? fixed_group(p, int(state_len), n_tok) : 0;
+  shape[0] = p.G;
+  shape[1] = rows_per_launch(p.limit, p.G);
+  shape[2] = G;
+  shape[3] = G == 0 ? 0 : G == 1 ? p.rows : rows_per_launch(p.limit, G);
 }
 
 int64_t chain_scratch_bytes(const kvm_layer &L, int64_t n_tok) {
@@ -2119,7 +2140,8 @@ hipError_t launch_chain(const kvm_layer &L, const kvm_seq &src, int64_t n_tok,
                          st, snaps, list, route_log, append_log, log_stride);
     return hipGetLastError();
   }
-  const int row_batch = p.limit / G / 8 * 8;  // rows a launch keeps resident, one group per XCD each
+  const int row_batch = rows_per_launch(p.limit, G);
+  if (row_batch <= 0) return hipErrorInvalidConfiguration;
   for (int row0 = 0; row0 < rows; row0 += row_batch) {
     const int nrows = std::min(row_batch, rows - row0);
     // Barrier counters and the abort flag start at zero in every launch.

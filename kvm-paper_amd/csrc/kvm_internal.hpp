@@ -123,6 +123,10 @@ struct ChainPlan {
 };
 // False when the shape does not fit the chain (the per-update kernels then run).
 bool chain_plan(const kvm_layer &L, int64_t n_tok, int64_t max_slots, ChainPlan *p);
+// The same for a device of `cus` compute units (host arithmetic only).
+bool chain_plan_on(int64_t cus, const kvm_layer &L, int64_t n_tok, int64_t max_slots, ChainPlan *p);
+// Workgroups per row and rows per launch, of batches with appends and of those without at state_len slots.
+void chain_shape(const ChainPlan &p, int64_t state_len, int64_t n_tok, int32_t *shape);
 // Whether a batch may use the chains without appends (slot-owner or one
 // workgroup per row): no appends, one state length, and a fitting group size.
 bool chain_fixed_ok(const ChainPlan &p, const ChainList &list, int64_t n_tok);

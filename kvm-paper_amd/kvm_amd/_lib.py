@@ -158,6 +158,7 @@ SIGNATURES = {
     "kvm_struct_size": (_i64, [ctypes.c_int]),
     "kvm_last_error": (ctypes.c_char_p, []),
     "kvm_prefill_workspace_bytes": (_i64, [_P(KvmPrefillDesc)]),
+    "kvm_chain_shape": (ctypes.c_int, [_P(KvmLayer), _i64, _i64, _i64, _P(ctypes.c_int32)]),
     "kvm_prefill": (ctypes.c_int, [_P(KvmPrefillDesc), _vp]),
     "kvm_prefill_backward_workspace_bytes": (_i64, [_P(KvmPrefillBwdDesc)]),
     "kvm_prefill_backward": (ctypes.c_int, [_P(KvmPrefillBwdDesc), _vp]),

@@ -199,6 +199,37 @@ def test_workspace_queries():
     assert lib.kvm_update_workspace_bytes(ctypes.byref(bad), 64) == -1
 
 
+def _chain_shape(max_state_len, state_len, compute_units, **kw):
+    lib = _lib()
+    layer, keep = _layer(**kw)
+    shape = (ctypes.c_int32 * 4)(-1, -1, -1, -1)
+    assert lib.kvm_chain_shape(ctypes.byref(layer), max_state_len, state_len, compute_units, shape) == 0
+    return tuple(shape)
+
+
+@pytest.mark.parametrize("cus", [8, 31, 32, 38, 63, 64, 76, 128, 256, 304])
+def test_chain_groups_fit_the_device(cus):
+    """Every group that a launch is given rows for is one that the device holds
+    eight of, whatever group the plan itself took."""
+    limit = min(cus, 256)
+    for D in (64, 128):
+        for C in (16, 64, 100, 256, 512, 1000):
+            for S in (16, C, 200, 512, 513, 1024, 2000):
+                for batch in (1, 2, 5, 16, 64):
+                    g, per, fg, fper = _chain_shape(max(S, C), S, cus, batch=batch, q_heads=4, kv_heads=4, head_dim=D,
+                                                    value_dim=D, chunk_len=C)
+                    what = (cus, D, C, S, batch, g, per, fg, fper)
+                    assert g in (0, 4, 8, 16) and fg in (0, 1, 4, 8, 16), what
+                    for group, rows in ((g, per), (fg, fper)):
+                        if group > 1:
+                            assert rows >= 8 and rows % 8 == 0 and rows * group <= limit, what
+                    if g == 0:
+                        assert (per, fg, fper) == (0, 0, 0), what
+    # 32 compute units hold eight groups of four members and no group of eight.
+    assert _chain_shape(256, 256, 32, batch=1, q_heads=4, kv_heads=4, chunk_len=256)[2] in (1, 4)
+    assert _chain_shape(1024, 1024, 32, batch=1, q_heads=4, kv_heads=4, chunk_len=256)[:3] == (4, 8, 0)
+
+
 def test_prefill_schedule_validation():
     lib = _lib()
     from kvm_amd import _lib as L
