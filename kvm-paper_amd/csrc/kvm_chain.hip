@@ -187,6 +187,37 @@ __device__ __forceinline__ int route_key_slot(uint64_t key) {
   return key ? int(0xffffffffu - uint32_t(key)) : -1;
 }
 
+// The running first maximum (best, from -inf on, and its slot) against a
+// lane's four consecutive slots from j0 on; equal scores go to the earlier
+// slot.  A tree of comparisons, with independent chains per token tile, where
+// all four count and none is NaN, which would stand for its neighbours ...
+__device__ __forceinline__ void keep_max4(const f32x4 &a, int j0, float &best, int &slot) {
+  const bool t1 = a[1] > a[0], t3 = a[3] > a[2];
+  const float v01 = t1 ? a[1] : a[0], v23 = t3 ? a[3] : a[2];
+  const int i01 = t1 ? 1 : 0, i23 = t3 ? 3 : 2;
+  const bool th = v23 > v01;
+  const float vh = th ? v23 : v01;
+  const bool take = vh > best;
+  best = take ? vh : best;
+  slot = take ? j0 + (th ? i23 : i01) : slot;
+}
+// ... and slot by slot over those in [lo, hi), where a NaN never wins.
+__device__ __forceinline__ void scan_max4(const f32x4 &a, int j0, int lo, int hi, float &best, int &slot) {
+#pragma unroll
+  for (int x = 0; x < 4; ++x) {
+    const float sc = (j0 + x >= lo) && (j0 + x < hi) ? a[x] : -INFINITY;
+    const bool take = sc > best;
+    best = take ? sc : best;
+    slot = take ? j0 + x : slot;
+  }
+}
+// Whether a block of 16 slots from jb on needs the scan: slots outside
+// [lo, hi), or a NaN key (a: the first operand of the block's keys; a key row
+// is a LayerNorm's output, NaN in every feature or in none).  Wave-uniform.
+__device__ __forceinline__ bool needs_scan(const uint4 &a, int jb, int lo, int hi) {
+  return jb < lo || jb + 16 > hi || __any((a.x & 0x7fffu) > 0x7f80u);
+}
+
 // LDS byte address of a __shared__ object (wave-uniform).
 typedef __attribute__((address_space(3))) void lds_void;
 template <typename T>
@@ -452,31 +483,25 @@ __global__ __launch_bounds__(kChainThreads) void k_chain(
             accs[tt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(a[ks]), as_bf16x8(bx[tt][ks]), accs[tt], 0,
                                                                0, 0);
         const int j0 = jb + (lane >> 4) * 4;
-        if (jb < lo || jb + 16 > hi) {  // slots outside [lo, hi) never count
+        if constexpr (NOVELTY) {
+          if (jb + 16 > hi) {  // slots past hi never count (lo is 0)
 #pragma unroll
-          for (int tt = 0; tt < 4; ++tt)
+            for (int tt = 0; tt < 4; ++tt)
 #pragma unroll
-            for (int x = 0; x < 4; ++x)
-              accs[tt][x] = (j0 + x >= lo) & (j0 + x < hi) ? accs[tt][x] : -INFINITY;
-        }
-#pragma unroll
-        for (int tt = 0; tt < 4; ++tt) {
-          const f32x4 acc = accs[tt];
-          if constexpr (NOVELTY) {
-            // The rounding is monotone, so the maximum may be taken first.
-            best[tt] = fmaxf(best[tt], fmaxf(fmaxf(acc[0], acc[1]), fmaxf(acc[2], acc[3])));
-          } else {
-            // The lane's four slots as a tree (the earlier keeps ties), then
-            // against the running maximum: the first maximum in slot order.
-            const bool t1 = acc[1] > acc[0], t3 = acc[3] > acc[2];
-            const float v01 = t1 ? acc[1] : acc[0], v23 = t3 ? acc[3] : acc[2];
-            const int i01 = t1 ? 1 : 0, i23 = t3 ? 3 : 2;
-            const bool th = v23 > v01;
-            const float vh = th ? v23 : v01;
-            const bool take = vh > best[tt];
-            best[tt] = take ? vh : best[tt];
-            bidx[tt] = take ? j0 + (th ? i23 : i01) : bidx[tt];
+              for (int x = 0; x < 4; ++x) accs[tt][x] = j0 + x < hi ? accs[tt][x] : -INFINITY;
           }
+#pragma unroll
+          for (int tt = 0; tt < 4; ++tt) {
+            // The rounding is monotone, so the maximum may be taken first.
+            const f32x4 acc = accs[tt];
+            best[tt] = fmaxf(best[tt], fmaxf(fmaxf(acc[0], acc[1]), fmaxf(acc[2], acc[3])));
+          }
+        } else if (needs_scan(a[0], jb, lo, hi)) {
+#pragma unroll
+          for (int tt = 0; tt < 4; ++tt) scan_max4(accs[tt], j0, lo, hi, best[tt], bidx[tt]);
+        } else {
+#pragma unroll
+          for (int tt = 0; tt < 4; ++tt) keep_max4(accs[tt], j0, best[tt], bidx[tt]);
         }
       }
 #pragma unroll
@@ -1481,8 +1506,7 @@ __global__ __launch_bounds__(kChainThreads) void k_chain_fixed(
         for (int ks = 0; ks < KS; ++ks)
           a[ks] = *reinterpret_cast<const uint4 *>(
               &own_k[(lt + (lane & 15)) * STR + ks * 32 + (lane >> 4) * 8]);
-        // Only a block holding sink slots or slots >= S needs the mask.
-        const bool masked = jb < protect || jb + 16 > S;
+        const bool scan = needs_scan(a[0], jb, protect, S);
         // k-steps outermost: the four token tiles' accumulations interleave
         // (each still sums its k-steps in order).
         f32x4 accs[4];
@@ -1505,35 +1529,12 @@ __global__ __launch_bounds__(kChainThreads) void k_chain_fixed(
           __builtin_amdgcn_sched_barrier(0);
         }
         const int j0 = jb + (lane >> 4) * 4;  // slot of acc[0]
-        if (masked) {
+        if (scan) {
 #pragma unroll
-          for (int tt = 0; tt < 4; ++tt) {
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-              const int j = j0 + i;
-              const float sc = ((j >= protect) && (j < S)) ? accs[tt][i] : -INFINITY;
-              const bool take = sc > best[tt];
-              best[tt] = take ? sc : best[tt];
-              bidx[tt] = take ? j : bidx[tt];
-            }
-          }
+          for (int tt = 0; tt < 4; ++tt) scan_max4(accs[tt], j0, protect, S, best[tt], bidx[tt]);
         } else {
-          // The lane's four slots as a tree (the earlier slot keeps ties),
-          // then against the running maximum: the same first maximum as a
-          // scan in slot order, with independent chains per token tile.
 #pragma unroll
-          for (int tt = 0; tt < 4; ++tt) {
-            const f32x4 acc = accs[tt];
-            const bool t1 = acc[1] > acc[0], t3 = acc[3] > acc[2];
-            const float v01 = t1 ? acc[1] : acc[0], v23 = t3 ? acc[3] : acc[2];
-            const int i01 = t1 ? 1 : 0, i23 = t3 ? 3 : 2;
-            const bool th = v23 > v01;
-            const float vh = th ? v23 : v01;
-            const int ih = th ? i23 : i01;
-            const bool take = vh > best[tt];
-            best[tt] = take ? vh : best[tt];
-            bidx[tt] = take ? j0 + ih : bidx[tt];
-          }
+          for (int tt = 0; tt < 4; ++tt) keep_max4(accs[tt], j0, best[tt], bidx[tt]);
         }
       }
       KVM_TS(12);
@@ -1760,24 +1761,12 @@ __global__ __launch_bounds__(kRowThreads) void k_chain_row(
             accs[tt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(a[ks]), as_bf16x8(bx[tt][ks]), accs[tt], 0,
                                                                0, 0);
         const int j0 = jb + (lane >> 4) * 4;
-        const bool masked = jb < protect || jb + 16 > S;
+        if (needs_scan(a[0], jb, protect, S)) {
 #pragma unroll
-        for (int tt = 0; tt < TT; ++tt) {
-          f32x4 acc = accs[tt];
-          if (masked) {  // sink slots and slots past S never win
+          for (int tt = 0; tt < TT; ++tt) scan_max4(accs[tt], j0, protect, S, best[tt], bidx[tt]);
+        } else {
 #pragma unroll
-            for (int x = 0; x < 4; ++x) acc[x] = (j0 + x >= protect) & (j0 + x < S) ? acc[x] : -INFINITY;
-          }
-          // The lane's four slots as a tree (the earlier keeps ties), then
-          // against the running maximum: the first maximum in slot order.
-          const bool t1 = acc[1] > acc[0], t3 = acc[3] > acc[2];
-          const float v01 = t1 ? acc[1] : acc[0], v23 = t3 ? acc[3] : acc[2];
-          const int i01 = t1 ? 1 : 0, i23 = t3 ? 3 : 2;
-          const bool th = v23 > v01;
-          const float vh = th ? v23 : v01;
-          const bool take = vh > best[tt];
-          best[tt] = take ? vh : best[tt];
-          bidx[tt] = take ? j0 + (th ? i23 : i01) : bidx[tt];
+          for (int tt = 0; tt < TT; ++tt) keep_max4(accs[tt], j0, best[tt], bidx[tt]);
         }
       }
 #pragma unroll

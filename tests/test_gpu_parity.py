@@ -1071,3 +1071,35 @@ def test_appending_chain_matches_per_update_kernels(lib, monkeypatch, B, Hkv, Tn
     T.log(f"[chain-append] {plan.n_updates} updates, {plan.initial_state_len} -> {plan.final_state_len} slots")
     for key in ("append_log", "route_log", "out", "state_k", "state_v", "state_vlen", "state_k_attn", "state_v_attn"):
         assert torch.equal(res["1"][key], res["0"][key]), key
+
+
+@pytest.mark.parametrize("B,Hkv,Tn,D,C,mode", [
+    (1, 4, 1400, 128, 128, "power_law"),   # appending chain
+    (2, 16, 1300, 64, 96, "power_law"),
+    (1, 4, 1500, 128, 128, "fixed"),       # slot-owner chain
+    (9, 33, 1000, 64, 96, "fixed"),        # one workgroup per row
+])
+def test_chains_with_nan_keys_match_per_update_kernels(lib, monkeypatch, B, Hkv, Tn, D, C, mode):
+    """A slot whose key is NaN takes no token and hides none of its neighbours:
+    routes and append sets equal the per-update kernels'."""
+    T.log(f"[chain-nan] B{B} Hkv{Hkv} T{Tn} D{D} C{C} {mode}")
+    cfg = T.mixer_config(Hkv, Hkv, D, C, mode=mode, sink=1, min_len=C, n_max=8, factor=16.0)
+    gen = torch.Generator().manual_seed(3)
+    m = T.make_mixer(cfg, (1 + 0.1 * torch.randn(D, generator=gen)).bfloat16(),
+                     (0.1 * torch.randn(D, generator=gen)).bfloat16(), torch.ones(Hkv), torch.ones(Hkv))
+    q, k, v, g = _random_inputs(B, Hkv, Hkv, Tn, D, 41)
+    for t in (4, 21, 34, 47):  # initial slots in every place of a lane's four
+        k[:, :, t, -1] = math.nan
+    if mode != "fixed":
+        k[:, :, 2 * C + 5, -1] = math.nan  # appended
+    q, k, v, g = (t.to(DEV) for t in (q, k, v, g))
+    res = {}
+    for chain in ("1", "0"):
+        monkeypatch.setenv("KVM_AMD_CHAIN", chain)
+        with torch.no_grad():
+            res[chain] = m.prefill_raw(q, k, v, g, route_log=True)
+        torch.cuda.synchronize()
+    assert bool(res["0"]["state_k"].isnan().any())
+    for key in ("append_log", "route_log", "state_k", "state_v", "state_vlen"):
+        a, b = res["1"][key], res["0"][key]
+        assert bool(((a == b) | (a.isnan() & b.isnan())).all()), key
