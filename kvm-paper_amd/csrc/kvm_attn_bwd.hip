@@ -479,8 +479,8 @@ void k_attn_bwd_dkdv(kvm_layer L, BwdArgs A, int kblocks, ChunkTable table) {
   const int64_t kp = kr;  // the lane's key (column lane%16 of every C tile)
   // Query t sees key p iff, in the window, p <= t < (p/C + n) C (the chunk of
   // t starts its window at or before p), and in a snapshot always.  Kept as
-  // offsets from tq_lo: [vis0, vis1) of the lane's key (empty for a key past
-  // the range), [all0, all1) seen by every key of the wave, [any0, any1) by
+  // offsets from tq_lo: vis_n queries from vis0 on for the lane's key (none for
+  // a key past the range), [all0, all1) seen by every key of the wave, [any0, any1) by
   // some.  Following the chunk of every query block instead took two 64-bit
   // scalar divisions per block and wave.
   const int64_t kw = kb0 + wave * 16;  // the wave's first key
@@ -551,7 +551,9 @@ void k_attn_bwd_dkdv(kvm_layer L, BwdArgs A, int kblocks, ChunkTable table) {
           for (int i = 0; i < 4; ++i) {
             const bool vis = !mask.value || uint32_t(t0 + qr + i - vis0) < vis_n;
             p[i] = vis ? __builtin_amdgcn_exp2f(__builtin_fmaf(s[i], sc, -lv[i])) : 0.f;
-            d[i] = p[i] * (dp[i] - dv4[i]) * dsc;
+            // Not p * ...: a hidden query's dP or delta may be infinite, and the
+            // statistics past a ragged block's end are those of an earlier block.
+            d[i] = vis ? p[i] * (dp[i] - dv4[i]) * dsc : 0.f;
           }
           pp[q2][0] = pack_bf16x2(p[0], p[1]);
           pp[q2][1] = pack_bf16x2(p[2], p[3]);

@@ -363,3 +363,50 @@ def test_state_backward_rounds_tokens_that_no_slot_took(B, Hkv, D, C, Tn):
         assert not wrong, f"{name} rows (batch, head, token) {wrong[:8]}"
     for t in bad:
         assert torch.equal(dk[:, :, t], win[0][:, :, t]) and not bool(dgate[:, :, t].any())
+
+
+@pytest.mark.parametrize("Hq,Hkv,D,C,Tn", [(4, 2, 128, 48, 331), (2, 2, 64, 80, 405), (2, 1, 128, 192, 705)])
+def test_attention_backward_reaches_seen_keys_only(Hq, Hkv, D, C, Tn):
+    """A gradient of one query alone: every key outside its window, every
+    snapshot but its chunk's and every other query's row are exactly zero.
+    With an infinite one the keys that the query does not see keep a zero key
+    gradient (a hidden pair contributes nothing, whatever its dP is)."""
+    if not torch.cuda.is_available():
+        pytest.skip("needs an MI355X")
+    from kvm_amd import training
+
+    T.log(f"[backward visibility] Hq{Hq} Hkv{Hkv} D{D} C{C} T{Tn}")
+    m = T.make_mixer(T.mixer_config(Hq, Hkv, D, C, rope=16), torch.ones(D), torch.zeros(D), torch.ones(Hq),
+                     torch.ones(Hq))
+    gen = torch.Generator().manual_seed(8)
+    q, k, v = (torch.randn(1, h, Tn, D, generator=gen).bfloat16().to(DEV) for h in (Hq, Hkv, Hkv))
+    g = torch.ones(1, Hkv, Tn, 1).bfloat16().to(DEV)
+    with torch.no_grad():
+        res = m.prefill_raw(q, k, v, g, route_log=True, keep_snapshots=True, want_lse=True)
+    plan, n = res["plan"], m.config.n_bswa_chunks
+    row = torch.randn(Hq, D, generator=gen).bfloat16().to(DEV)
+    for t in sorted({0, 31, 63, 64, C - 1, C, 2 * C - 1, 2 * C, 2 * C + 5, 3 * C - 1, 3 * C, Tn - 9, Tn - 1}):
+        chunk = t // C
+        seen = torch.zeros(Tn, dtype=torch.bool, device=DEV)
+        seen[max(0, (chunk - n + 1) * C):t + 1] = True
+        for inf in (False, True):
+            dout = torch.zeros(1, Tn, Hq, D, device=DEV, dtype=torch.bfloat16)
+            dout[0, t] = row
+            if inf:
+                dout[0, t, :, 0] = math.inf
+            dq, dk, dv, dsk, dsv, _, _ = training.attention_backward(m, q, k, v, g, res, dout)
+            other = torch.arange(Tn, device=DEV) != t
+            assert not bool(dq[:, :, other].ne(0).any()), f"dq of query {t}"
+            hit = dk[:, :, ~seen].ne(0).any(-1).nonzero().tolist()  # NaN is not zero
+            assert not hit, f"dk (batch, head, hidden key) {hit[:4]} of query {t}, infinite {inf}"
+            if inf:
+                continue
+            assert not bool(dv[:, :, ~seen].ne(0).any()), f"dv of query {t}"
+            assert bool(dv[:, :, seen].abs().amax(-1).gt(0).all()), f"a key that query {t} sees has no dv"
+            own = plan.chunk_snapshot[chunk] if chunk >= n else -1
+            for s in range(dsv.size(0)):
+                S = ([plan.initial_state_len] + [a + b for a, b in zip(plan.upd_state_before, plan.upd_n_append)])[s]
+                if s == own:
+                    assert bool(dsv[s, :, :S].abs().amax(-1).gt(0).all())
+                elif s in [plan.chunk_snapshot[c] for c in range(n, plan.n_chunks)]:
+                    assert not bool(dsv[s].ne(0).any()) and not bool(dsk[s].ne(0).any()), f"snapshot {s} of query {t}"
