@@ -36,12 +36,13 @@
 // line: the scores of the second half issue before the output products of the
 // first, so a wave has independent matrix work under its exponentials (at two
 // waves per SIMD the kernels wait on their own chains, not on LDS, L2 or the
-// matrix units: 26 - 44 % matrix-busy, 46 % of the wave cycles of the window
-// kernel waiting before).  Measured at 32768 tokens x 32 heads of 128: dq 1297
-// -> 1165 us, window dk/dv 1604 -> 1206, snapshots 779 -> 830; 2 x 16 (4 kv) heads of 64, 4099 tokens: dq 110
-// -> 79, window 45 -> 33, snapshots 87 -> 76.  32 keys per dk/dv wave, half
-// the LDS reads, were slower (2332 us: one wave per SIMD; 45 -> 64 us at
-// D = 64).
+// matrix units).  Measured at 32768 tokens x 32 heads of 128, with one path
+// for every block before and now: dq 1297 -> 1165 us, window dk/dv 1660 ->
+// 1170, snapshots 805 -> 807 (a half at a time there: 1030); 8 x 6 heads, 8192
+// tokens: window 404 -> 295, snapshots 206 -> 201; 2 x 16 (4 kv) heads of 64,
+// 4099 tokens: dq 110 -> 79, window 46 -> 33, snapshots 90 -> 75.  32 keys per
+// dk/dv wave, half the LDS reads, were slower (2332 us: one wave per SIMD; 45
+// -> 64 us at D = 64).
 
 #include <type_traits>
 
@@ -80,8 +81,8 @@ __device__ __forceinline__ int xcd_logical(int bid, int N) {
 // compiler keeps too few LDS reads in flight for two waves per SIMD.  The
 // products also run at a raised wave priority, so that the other wave's
 // exponentials fill their gaps and not the other way round.  32768 tokens x 32
-// heads: window 1464 us with neither, 1339 with the priority, 1206 with both;
-// snapshots 942 / 876 / 830.  At D = 64, with four waves per SIMD, neither
+// heads, when each was added: window 1464 us with neither, 1339 with the
+// priority, 1206 with both; snapshots 942 / 876 / 830.  At D = 64, with four waves per SIMD, neither
 // gains (priority: snapshots 76 -> 81 us; grouped reads: 33 -> 34, 76 -> 77).
 __device__ __forceinline__ void interleave_products() {
   constexpr int kMfma = 0x8, kLdsRead = 0x100;
@@ -532,16 +533,24 @@ void k_attn_bwd_dkdv(kvm_layer L, BwdArgs A, int kblocks, ChunkTable table) {
       // P and dS (scaled by tau / sqrt(D)) of the 32 queries of step hb in the
       // B-operand layout: lane holds queries qt*16 + 4*(lane/16) + i of key lane%16.
       auto scores = [&](int hb, auto mask, bf16x8 &pb, bf16x8 &db) {
+        // Both query tiles' products before either's exponentials: a tile at a
+        // time left the snapshots' blocks 1 % and the window's 2 % slower.
         uint32_t pp[2][2], pd[2][2];
+        f32x4 st[2], dpt[2];
 #pragma unroll
         for (int q2 = 0; q2 < 2; ++q2) {
           const int qt = 2 * hb + q2;
-          f32x4 s = f32x4{0.f, 0.f, 0.f, 0.f}, dp = f32x4{0.f, 0.f, 0.f, 0.f};
+          st[q2] = dpt[q2] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
           for (int ks = 0; ks < KS; ++ks) {
-            s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(row_frag(qimg, lo, qt, ks), kf[ks], s, 0, 0, 0);
-            dp = __builtin_amdgcn_mfma_f32_16x16x32_bf16(row_frag(dimg, lo, qt, ks), vf[ks], dp, 0, 0, 0);
+            st[q2] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(row_frag(qimg, lo, qt, ks), kf[ks], st[q2], 0, 0, 0);
+            dpt[q2] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(row_frag(dimg, lo, qt, ks), vf[ks], dpt[q2], 0, 0, 0);
           }
+        }
+#pragma unroll
+        for (int q2 = 0; q2 < 2; ++q2) {
+          const int qt = 2 * hb + q2;
+          const f32x4 s = st[q2], dp = dpt[q2];
           const int qr = qt * 16 + (lane >> 4) * 4;  // block-relative query of i = 0
           const float4 l4 = *reinterpret_cast<const float4 *>(lse_s + qr);
           const float4 d4 = *reinterpret_cast<const float4 *>(dl_s + qr);
