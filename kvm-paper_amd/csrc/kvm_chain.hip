@@ -92,7 +92,7 @@ namespace {
 __host__ __device__ inline int append_red_bytes(int n_tok, int own_cap) {
   int ntg = 64;
   while (ntg < n_tok) ntg <<= 1;
-  const int scan = (ntg < 512 ? 512 : ntg) * 8, lists = (n_tok + 63) / 64 * own_cap * 2;
+  const int scan = (ntg < 512 ? 512 : ntg) * 8, lists = (n_tok + 63) / 64 * own_cap;
   return ((scan > lists ? scan : lists) + 15) & ~15;
 }
 // ... then off / cnt [own_cap] and sorted / apos [n_tok].
@@ -100,7 +100,11 @@ __host__ __device__ inline int append_lds_bytes(int n_tok, int own_cap) {
   return append_red_bytes(n_tok, own_cap) + 4 * own_cap + 4 * n_tok;
 }
 
-constexpr int kAppendDynLds = 44 * 1024;  // beside the attention keys (OwnLds)
+// Beside the attention keys (OwnLds): room for 2144 own slots per member at
+// 1024 tokens per update, 3744 at 512 (29952 slots with eight members).  32
+// rows of 128, C 512, up to 18892 slots: 11.8 ms a prefill, 18.3 on the
+// per-update kernels, which states past the tables run on.
+constexpr int kAppendDynLds = 46 * 1024;
 constexpr int kChainThreads = 512;
 constexpr int kChainWaves = kChainThreads / 64;
 constexpr int kChainTok = 64;        // tokens per member at most
@@ -318,11 +322,11 @@ __global__ __launch_bounds__(kChainThreads) void k_chain(
   __shared__ int ok_lds;
   __shared__ float ln_w[D], ln_b[D];  // ln_s_k parameters (LDS: no wait on global loads)
   // [slot group][token] maxima of a scan (8 bytes each); in their place, the
-  // lists' counts [64 tokens][own_cap].  Then off / cnt [own_cap], sorted and
-  // apos [n_tok] (append_lds_bytes).
+  // lists' counts [64 tokens][own_cap], at most 64 each.  Then off / cnt
+  // [own_cap], sorted and apos [n_tok] (append_lds_bytes).
   extern __shared__ __attribute__((aligned(16))) uint64_t red[];
-  uint16_t *const wsc = reinterpret_cast<uint16_t *>(red);
-  uint16_t *const off = wsc + append_red_bytes(n_tok, own_cap) / 2, *const cnt = off + own_cap;
+  uint8_t *const wsc = reinterpret_cast<uint8_t *>(red);
+  uint16_t *const off = reinterpret_cast<uint16_t *>(wsc + append_red_bytes(n_tok, own_cap)), *const cnt = off + own_cap;
   uint16_t *const sorted = cnt + own_cap;                              // tokens of my slots, slot by slot
   int16_t *const apos = reinterpret_cast<int16_t *>(sorted + n_tok);   // append position of a token or -1
 
@@ -699,7 +703,7 @@ __global__ __launch_bounds__(kChainThreads) void k_chain(
     const int nvw = (n_tok + 63) >> 6;
     const int nblk = (s_after + 15) >> 4;
     const int nown = member < nblk ? ((nblk - 1 - member) / G + 1) * 16 : 0;  // my local slots in use
-    for (int e = tid; e < nvw * own_cap; e += kChainThreads) wsc[e] = 0;
+    for (int e = tid; e < nvw * own_cap / 4; e += kChainThreads) reinterpret_cast<uint32_t *>(wsc)[e] = 0;
     constexpr int NT = 2;  // tokens per thread (n_tok <= 1024)
     int loc[NT], rank[NT];
     uint64_t pkey[NT];
@@ -741,21 +745,16 @@ __global__ __launch_bounds__(kChainThreads) void k_chain(
         }
         rank[x] = int(__builtin_amdgcn_mbcnt_hi(uint32_t(eq >> 32), __builtin_amdgcn_mbcnt_lo(uint32_t(eq), 0u)));
         if (mine) loc[x] = l;
-        if (mine && rank[x] == 0) wsc[(x * kChainWaves + wave) * own_cap + l] = uint16_t(__popcll(eq));
+        if (mine && rank[x] == 0) wsc[(x * kChainWaves + wave) * own_cap + l] = uint8_t(__popcll(eq));
       }
     }
     __syncthreads();
-    // Exclusive prefix: over the token groups of each slot's counts (in
-    // place), then over the slots, kChainThreads of them at a time.
+    // Exclusive prefix over the slots' counts, kChainThreads slots at a time.
     for (int e0 = 0, run = 0; e0 < nown; e0 += kChainThreads) {
       const int e = e0 + tid;
       int tot = 0;
       if (e < nown)
-        for (int w = 0; w < nvw; ++w) {
-          const int n = wsc[w * own_cap + e];
-          wsc[w * own_cap + e] = uint16_t(tot);
-          tot += n;
-        }
+        for (int w = 0; w < nvw; ++w) tot += wsc[w * own_cap + e];
       int incl = tot;
 #pragma unroll
       for (int o = 1; o < 64; o <<= 1) {
@@ -778,9 +777,11 @@ __global__ __launch_bounds__(kChainThreads) void k_chain(
     }
 #pragma unroll
     for (int x = 0; x < NT; ++x)
-      if (x * kChainThreads < n_tok && loc[x] >= 0)
-        sorted[off[loc[x]] + wsc[(x * kChainWaves + wave) * own_cap + loc[x]] + rank[x]] =
-            uint16_t(x * kChainThreads + tid);
+      if (x * kChainThreads < n_tok && loc[x] >= 0) {
+        int at = off[loc[x]] + rank[x];  // behind the slot's tokens of earlier groups
+        for (int w = 0; w < x * kChainWaves + wave; ++w) at += wsc[w * own_cap + loc[x]];
+        sorted[at] = uint16_t(x * kChainThreads + tid);
+      }
     __syncthreads();
     KVM_TS_A(9);
 
@@ -2001,7 +2002,7 @@ bool chain_plan_on(int64_t cus, const kvm_layer &L, int64_t n_tok, int64_t max_s
     if ((G == 16 && groups * 16 > limit) || (G == 4 && groups * 8 <= limit)) continue;
     const int64_t tpw = ((n_tok + G - 1) / G + 15) / 16 * 16;
     const int64_t own_cap = ((max_slots + 15) / 16 + G - 1) / G * 16;
-    if (tpw > kChainTok || rows_per_launch(limit, G) == 0 || n_tok < 1 || max_slots > 32768) continue;
+    if (tpw > kChainTok || rows_per_launch(limit, G) == 0 || n_tok < 1 || max_slots > 65536) continue;
     const int64_t dyn = append_lds_bytes(int(n_tok), int(own_cap));
     if (dyn > kAppendDynLds) continue;
     p->fixed = false;

@@ -1103,3 +1103,43 @@ def test_chains_with_nan_keys_match_per_update_kernels(lib, monkeypatch, B, Hkv,
     for key in ("append_log", "route_log", "state_k", "state_v", "state_vlen"):
         a, b = res["1"][key], res["0"][key]
         assert bool(((a == b) | (a.isnan() & b.isnan())).all()), key
+
+
+def _chain_shape(lib, m, B, max_state_len, state_len):
+    """(workgroups per row of batches with appends, of those without)."""
+    import ctypes
+
+    shape = (ctypes.c_int32 * 4)()
+    assert lib.kvm_chain_shape(m._layer_struct(B, torch.device(DEV)).ref(), max_state_len, state_len, 0, shape) == 0
+    return shape[0], shape[2]
+
+
+def _chain_against_per_update(lib, monkeypatch, m, inputs):
+    q, k, v, g = (t.to(DEV) for t in inputs)
+    res = {}
+    for chain in ("1", "0"):
+        monkeypatch.setenv("KVM_AMD_CHAIN", chain)
+        with torch.no_grad():
+            res[chain] = m.prefill_raw(q, k, v, g, route_log=True)
+        torch.cuda.synchronize()
+    for key in ("append_log", "route_log", "out", "state_k", "state_v", "state_vlen", "state_k_attn", "state_v_attn"):
+        assert torch.equal(res["1"][key], res["0"][key]), key
+    return res["1"]["plan"]
+
+
+@pytest.mark.parametrize("B,Hkv,Tn,D,C,group", [
+    (1, 17, 21000, 64, 512, 8),    # 8 token groups, about 2300 own slots per member
+    (1, 1, 23600, 64, 1024, 16),   # 16 token groups, about 1270 own slots
+])
+def test_appending_chain_of_large_states_matches_per_update_kernels(lib, monkeypatch, B, Hkv, Tn, D, C, group):
+    """States whose slot lists fill the appending chain's tables at wide chunks
+    (nine tenths of the tokens become slots)."""
+    T.log(f"[chain-large] B{B} Hkv{Hkv} T{Tn} D{D} C{C}")
+    cfg = T.mixer_config(Hkv, Hkv, D, C, mode="power_law", min_len=C, n_max=64, factor=0.9, expo=1.0)
+    gen = torch.Generator().manual_seed(3)
+    m = T.make_mixer(cfg, (1 + 0.1 * torch.randn(D, generator=gen)).bfloat16(),
+                     (0.1 * torch.randn(D, generator=gen)).bfloat16(), torch.ones(Hkv), torch.ones(Hkv))
+    slots = m.make_plan(Tn).max_state_len
+    assert slots > 18300 and _chain_shape(lib, m, B, slots, slots)[0] == group
+    plan = _chain_against_per_update(lib, monkeypatch, m, _random_inputs(B, Hkv, Hkv, Tn, D, 43))
+    assert 0 < plan.upd_n_append[-1] < C

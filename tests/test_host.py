@@ -230,6 +230,23 @@ def test_chain_groups_fit_the_device(cus):
     assert _chain_shape(1024, 1024, 32, batch=1, q_heads=4, kv_heads=4, chunk_len=256)[:3] == (4, 8, 0)
 
 
+def test_appending_chain_holds_large_states():
+    """States that the appending chain's tables have to hold (12 bytes per slot
+    of a member beside 16 per token and a power of two of 8-byte sort keys in
+    48 KiB, the least that it ever took): it runs them at every chunk length."""
+    for C in (16, 40, 64, 100, 128, 200, 256, 300, 500, 512, 513, 700, 960, 1000, 1023, 1024):
+        for batch in (1, 4, 5, 8, 12, 64):  # x 4 rows
+            groups = (batch * 4 + 7) // 8 * 8
+            G = 16 if groups * 16 <= 256 else 8
+            if -(-(-(-C // G)) // 16) * 16 > 64:
+                continue
+            npow = 1 << (C - 1).bit_length()
+            slots = (48 * 1024 - 8 * npow - 16 * C - 4) // 12 * G
+            for S in (C, slots // 2, slots - 1, slots):
+                shape = _chain_shape(S, S, 256, batch=batch, q_heads=4, kv_heads=4, chunk_len=C)
+                assert shape[0] >= 4 and shape[1] >= 8, (C, batch, S, shape)
+
+
 def test_prefill_schedule_validation():
     lib = _lib()
     from kvm_amd import _lib as L
