@@ -1143,3 +1143,27 @@ def test_appending_chain_of_large_states_matches_per_update_kernels(lib, monkeyp
     assert slots > 18300 and _chain_shape(lib, m, B, slots, slots)[0] == group
     plan = _chain_against_per_update(lib, monkeypatch, m, _random_inputs(B, Hkv, Hkv, Tn, D, 43))
     assert 0 < plan.upd_n_append[-1] < C
+
+
+@pytest.mark.parametrize("B,Hkv,Tn,D,C,S,append_group,group", [
+    (8, 8, 1700, 128, 128, 512, 4, 4),    # four members of 128 own slots (96 staged rows)
+    (8, 8, 1700, 64, 128, 512, 4, 4),
+    (3, 8, 1700, 128, 128, 512, 8, 8),    # eight members of 64 own slots
+    (3, 8, 3100, 128, 256, 1000, 8, 8),   # of 128
+    (3, 8, 3100, 64, 256, 1000, 8, 8),
+    (16, 16, 900, 128, 64, 256, 4, 1),    # one workgroup per row, more slots than tokens
+    (16, 16, 1200, 64, 64, 500, 4, 1),
+    (1, 4, 1700, 64, 128, 512, 16, 16),
+])
+def test_chain_groups_match_per_update_kernels(lib, monkeypatch, B, Hkv, Tn, D, C, S, append_group, group):
+    """States that grow past a chunk and then stay: the appending chain, and
+    after it the chain without appends, each with the members per row that its
+    rule is to pick here."""
+    T.log(f"[chain-groups] B{B} Hkv{Hkv} T{Tn} D{D} C{C} {S} slots")
+    cfg = T.mixer_config(Hkv, Hkv, D, C, mode="fixed", min_len=S, n_max=-(-S // C))
+    gen = torch.Generator().manual_seed(3)
+    m = T.make_mixer(cfg, (1 + 0.1 * torch.randn(D, generator=gen)).bfloat16(),
+                     (0.1 * torch.randn(D, generator=gen)).bfloat16(), torch.ones(Hkv), torch.ones(Hkv))
+    assert _chain_shape(lib, m, B, S, S) == (append_group, group)
+    plan = _chain_against_per_update(lib, monkeypatch, m, _random_inputs(B, Hkv, Hkv, Tn, D, 47))
+    assert plan.final_state_len == S and sum(plan.upd_n_append) == S - C and plan.upd_n_append[-2:] == [0, 0]
