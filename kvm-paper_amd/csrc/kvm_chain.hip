@@ -326,7 +326,8 @@ __global__ __launch_bounds__(kChainThreads) void k_chain(
   // [own_cap], sorted and apos [n_tok] (append_lds_bytes).
   extern __shared__ __attribute__((aligned(16))) uint64_t red[];
   uint8_t *const wsc = reinterpret_cast<uint8_t *>(red);
-  uint16_t *const off = reinterpret_cast<uint16_t *>(wsc + append_red_bytes(n_tok, own_cap)), *const cnt = off + own_cap;
+  uint16_t *const off = reinterpret_cast<uint16_t *>(wsc + append_red_bytes(n_tok, own_cap));
+  uint16_t *const cnt = off + own_cap;
   uint16_t *const sorted = cnt + own_cap;                              // tokens of my slots, slot by slot
   int16_t *const apos = reinterpret_cast<int16_t *>(sorted + n_tok);   // append position of a token or -1
 
@@ -2022,26 +2023,34 @@ namespace {
 // Members per row of a chain without appends over S slots (1: k_chain_row),
 // or 0 when none fits.  Up to 16 rows: 16 members (chain_plan).  Above, more
 // members make an update shorter but fewer rows fit a launch, so the choice
-// is the least of launches x time per update.  Measured at D 128, C = S, us
-// per update for all rows, with 8 / 4 / 1 members:
-//   C 256   48 rows 18.5 / 12.1 / 28.0    96 rows 27.8 / 23.7 / 29.4
-//          128 rows 37.1 / 24.5 / 30.1   256 rows 74.4 / 48.4 / 32.8
-//   C 128   64 rows 13.7 /  7.7 / 15.3   128 rows 27.6 / 15.4 / 15.6
-//   C  64  128 rows 24.5 / 12.5 /  8.6
-// (C 512: one launch of 32 rows 11.7 with 8; 4 members would prep 128 tokens
-// each, which their staging rows do not hold.)  The lines below fit these: a
-// part that is latency, and a part that grows with the rows (tokens and
-// slots) a member works on.
+// is the least of launches x time per update.  Measured, us per update for all
+// rows, with 8 / 4 / 1 members (24 and 40 rows fill one launch of 8 and of 4):
+//   D    C    S     24 rows             40 rows              96 rows             256 rows
+//   128  256  256    7.8 /  9.8 / 21.1   15.0 / 10.1 / 22.0   23.7 / 20.5 / 22.7  63.5 / 47.8 / 30.6
+//   128  128  256    7.2 /  8.6 / 16.4   13.8 /  8.7 / 16.7   22.4 / 18.4 / 17.7  56.2 / 35.4 / 22.9
+//   128   64  256    6.9 /  8.1 / 13.7   13.1 /  8.4 / 13.9   20.4 / 17.1 / 14.8  52.0 / 33.4 / 16.6
+//   128  128  128    6.4 /  7.0 / 12.4   12.7 /  7.0 / 12.3   19.6 / 14.5 / 13.0  51.6 / 29.2 / 16.7
+//   128   16   16    5.8 /  5.6 /  6.7   11.5 /  5.7 /  6.7   17.5 / 11.5 /  6.9  45.7 / 23.1 /  7.0
+//    64  256  256    5.6 /  6.7 / 14.4   11.5 /  6.9 / 14.0   17.9 / 14.0 / 14.7  46.9 / 28.3 / 16.8
+//    64  128  512    6.2 /  8.7 / 15.6   12.3 /  8.9 / 15.5   19.0 / 18.1 / 16.7  49.5 / 35.4 / 17.1
+//    64  128  128    4.4 /  5.2 /  8.7   10.5 /  5.3 /  8.8   15.3 / 10.8 /  8.7  42.0 / 22.3 /  9.5
+//    64   16   16    4.7 /  4.4 /  6.3    9.4 /  4.7 /  6.6   14.4 /  9.4 /  6.6  37.8 / 18.8 /  6.7
+//    64  512  512    8.0 /   -  / 28.3   15.8 /   -  / 29.1   25.9 /   -  / 30.2  69.0 /   -  / 34.8
+// (C 512: 4 members would prep 128 tokens each, which their staging rows do
+// not hold.)  The lines below fit these and 18 more shapes: a part that is
+// latency, and parts that grow with the tokens and slots a member works on.
 int fixed_group(const ChainPlan &p, int S, int64_t n_tok) {
   if (n_tok > kFixedMaxTok) return 0;
   const int nblk = (S + 15) / 16;
   // Owned slots per member: up to 64 at G = 16, up to 128 below; at most kChainTok prep tokens;
   // and a launch that holds eight groups, which the plan has checked for its own G only.
   const auto fits = [&](int G) {
-    return rows_per_launch(p.limit, G) > 0 && (nblk + G - 1) / G * 16 <= (G == 16 ? 64 : kOwnMax) && (n_tok + G - 1) / G <= kChainTok;
+    return rows_per_launch(p.limit, G) > 0 && (nblk + G - 1) / G * 16 <= (G == 16 ? 64 : kOwnMax) &&
+           (n_tok + G - 1) / G <= kChainTok;
   };
   if (p.G == 16) return fits(16) ? 16 : 0;
-  const double work = double(n_tok + S) * p.head_dim / 128;
+  const bool wide = p.head_dim == 128;
+  const double tok = double(n_tok) * p.head_dim / 128, slots = double(S) * p.head_dim / 128;
   const auto launches = [&](int G) {
     const int per = G == 1 ? p.limit : rows_per_launch(p.limit, G);
     return double((p.rows + per - 1) / per);
@@ -2054,10 +2063,10 @@ int fixed_group(const ChainPlan &p, int S, int64_t n_tok) {
       least = us;
     }
   };
-  const int rmax = p.head_dim == 128 ? RowMax<128>::value : RowMax<64>::value;
-  if (fits(8)) offer(8, launches(8) * (5.2 + 0.0075 * work));
-  if (fits(4)) offer(4, launches(4) * (4.0 + 0.016 * work));
-  if (S <= rmax && n_tok <= rmax) offer(1, launches(1) * (1.5 + 0.058 * work));
+  const int rmax = wide ? RowMax<128>::value : RowMax<64>::value;
+  if (fits(8)) offer(8, launches(8) * ((wide ? 5.2 : 4.2) + 0.0066 * (tok + slots)));
+  if (fits(4)) offer(4, launches(4) * ((wide ? 4.7 : 4.2) + 0.0125 * (tok + slots)));
+  if (S <= rmax && n_tok <= rmax) offer(1, launches(1) * (5.2 + 0.05 * tok + 0.026 * slots));
   return best;
 }
 }  // namespace

@@ -247,6 +247,19 @@ def test_appending_chain_holds_large_states():
                 assert shape[0] >= 4 and shape[1] >= 8, (C, batch, S, shape)
 
 
+@pytest.mark.parametrize("D,C,S,rows,group", [
+    (64, 16, 16, 24, (4, 8)), (64, 32, 32, 24, (4, 8)), (128, 16, 16, 24, (4, 8)), (64, 16, 16, 64, (4,)),
+    (64, 128, 128, 24, (8,)), (64, 64, 64, 256, (1,)), (64, 64, 512, 96, (1,)), (64, 128, 512, 24, (8,)),
+    (128, 64, 256, 128, (1,)), (128, 128, 512, 64, (4,)), (128, 256, 256, 64, (4,)), (128, 256, 256, 256, (1,)),
+    (128, 128, 256, 24, (8,)), (64, 512, 512, 64, (8,)), (128, 512, 512, 32, (8,)), (128, 32, 256, 128, (1,)),
+])
+def test_chain_group_is_the_fastest_measured(D, C, S, rows, group):
+    """The choice where the measured group sizes are far apart (us per update
+    of all rows beside the rule), with chunks and states of different length."""
+    shape = _chain_shape(max(S, C), S, 256, batch=rows // 8, q_heads=8, kv_heads=8, head_dim=D, value_dim=D, chunk_len=C)
+    assert shape[2] in group, shape
+
+
 def test_prefill_schedule_validation():
     lib = _lib()
     from kvm_amd import _lib as L
