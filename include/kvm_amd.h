@@ -250,11 +250,12 @@ typedef struct kvm_state_bwd_desc {
   int64_t workspace_bytes;
 } kvm_state_bwd_desc;
 
+/* Of the descriptor's layer, max_state_len and n_updates. */
 int64_t kvm_state_backward_workspace_bytes(const kvm_state_bwd_desc *d);
 int kvm_state_backward(const kvm_state_bwd_desc *d, void *stream);
 /* The same with the sums rounded once into dk_out / dv_out (bf16 [B, Hkv,
- * seq_len, head_dim], 16-byte aligned), every token's row; dk / dv are only
- * read.  The updates' chunks must follow each other without gaps. */
+ * seq_len, head_dim], 16-byte aligned), every token's row (of a token that no
+ * slot took, its row of dk / dv); dk / dv are only read.  The updates' chunks must follow each other without gaps. */
 int kvm_state_backward_rounded(const kvm_state_bwd_desc *d, void *dk_out, void *dv_out, void *stream);
 
 /* The mixer's pre-boundary elementwise work on the q/k/v projections, for

@@ -873,14 +873,14 @@ int kvm_prefill(const kvm_prefill_desc *d, void *stream) {
     // leaving normally).
     if (const char *polls = getenv("KVM_AMD_CHAIN_POLLS"))
       cs.max_polls = unsigned(strtoul(polls, nullptr, 10));
-    // KVM_AMD_CHAIN_FIXED=0 keeps batches without appends on the token-split kernel.
+    // KVM_AMD_CHAIN_FIXED=0 keeps batches without appends on the appending chain (k_chain).
     const char *fixed_env = getenv("KVM_AMD_CHAIN_FIXED");
     const kvm::SnapRing ring{snap_k, snap_v, snap_stride, R, d->max_state_len};
     for (int64_t u = 0; u < d->n_updates;) {
       int64_t e = std::min({d->n_updates, u + int64_t(kvm::kChainMax), u + R});
       // A batch whose updates stop appending part-way (a growing budget that
       // reaches its cap) ends where they stop: the tail, whose state length
-      // no longer changes, runs on the slot-owner kernel in the next launch.
+      // no longer changes, runs on a chain without appends in the next launch.
       {
         int64_t tail = e;
         while (tail > u + 1 && d->upd_n_append[tail - 1] == 0 &&
@@ -905,7 +905,7 @@ int kvm_prefill(const kvm_prefill_desc *d, void *stream) {
       }
       kvm::ChainPlan bp = cp;
       bp.fixed = !(fixed_env && fixed_env[0] == '0') && kvm::chain_fixed_ok(cp, cl, C);
-      // The fixed chain's last batch writes the final attention rows itself.
+      // The chains without appends write the final attention rows themselves.
       cl.final_rows = int32_t(bp.fixed && e == d->n_updates && d->state.s_k_attn && d->state.s_v_attn);
       attn_rows_written = cl.final_rows != 0;
       KVM_HIP(kvm::launch_chain(L, d->kv, C, d->state, ring, cl, cs, bp, d->route_log,

@@ -108,7 +108,6 @@ constexpr int kAppendDynLds = 46 * 1024;
 constexpr int kChainThreads = 512;
 constexpr int kChainWaves = kChainThreads / 64;
 constexpr int kChainTok = 64;        // tokens per member at most
-constexpr int kTilesInFlight = 4;    // 16-slot tiles a wave loads at once
 constexpr int kCounterStride = 32;   // words between group counters (128 B)
 
 // Group barrier, split so that independent work can run between arriving
@@ -172,10 +171,6 @@ __device__ __forceinline__ uint4 l2_ld16(__amdgpu_buffer_rsrc_t r, int off) {
 }
 __device__ __forceinline__ uint32_t l2_ld4(__amdgpu_buffer_rsrc_t r, int off) {
   return __builtin_amdgcn_raw_buffer_load_b32(r, off, 0, kScopeDevice);
-}
-__device__ __forceinline__ uint64_t l2_ld8(__amdgpu_buffer_rsrc_t r, int off) {
-  const auto v = __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, kScopeDevice);
-  return uint64_t(v[0]) | (uint64_t(v[1]) << 32);
 }
 
 // Route key of a (score, slot) candidate: the per-update routing kernel's
@@ -1595,12 +1590,14 @@ __global__ __launch_bounds__(kChainThreads) void k_chain_fixed(
 // ---------------------------------------------------------------------------
 // The chain without appends when there are rows for every compute unit: one
 // workgroup per row, no exchange.  The slot-owner kernel above spends most of
-// an update on the latency of its exchange (8.3 us at 32 slots and 32 tokens
+// an update on the latency of its exchange (7.8 us at 32 slots and 32 tokens
 // per member, C 256, 256 slots), and runs 8 launches of 32 rows for 256 rows;
-// here a row's work is done in one place and every launch is full: 32.1 us per
-// update of 256 rows against 74.4.  Bound by VALU issue (the LayerNorms and
-// sums of C tokens and S slots): prep 4.2, route 8.8 (its key fragments from
-// LDS at 64 B per clock as much), lists 3.2, keys 7.4, values 1.7 + 6.9 us.
+// here a row's work is done in one place and every launch is full: less than
+// half the time at 256 rows (figures at fixed_group).  Bound by VALU issue
+// (the LayerNorms and sums of C tokens and S slots; VALU busy 80 % of the
+// compute units' busy cycles): of 32 us, prep 4.2, route 8.8 (its key
+// fragments from LDS at 64 B per clock as much), lists 3.2, keys 7.4, values
+// 1.7 + 6.9.
 // 16 waves of 128 registers: with 8 waves of 256 the phases but the route
 // were slower (34.8 us).
 //

@@ -88,7 +88,7 @@ constexpr int kChainMaxWorkgroups = 256;   // one 512-thread workgroup per CU
 struct ChainList {
   int32_t u0;     // update index of entry 0 (snapshot u0 -> u0 + 1, log offset)
   int32_t count;
-  int32_t final_rows;  // k_chain_fixed: also write the last snapshot's rows to the state's s_k_attn / s_v_attn
+  int32_t final_rows;  // k_chain_fixed, k_chain_row: also write the last snapshot's rows to the state's s_k_attn / s_v_attn
   int32_t tok_begin[kChainMax];
   int32_t state_before[kChainMax];
   int32_t n_append[kChainMax];
@@ -112,7 +112,7 @@ struct ChainScratch {
   unsigned max_polls;    // L2 polls a group wait makes before giving up
 };
 struct ChainPlan {
-  bool fixed;     // slot-owner routing (no appends in the batch)
+  bool fixed;     // no appends in the batch: k_chain_fixed, or k_chain_row for G = 1
   int G;          // workgroups per row
   int tpw;        // tokens per workgroup (multiple of 16, <= 64)
   int own_cap;    // owned slots per member at max_slots (whole blocks of 16)
