@@ -293,7 +293,8 @@ __global__ __launch_bounds__(kThreads) void k_route_sort(StateBwdArgs A, int ngr
 // Bound by VALU issue (the tokens' LayerNorms and chain rule, the slots'
 // local backward) and by memory: 2 waves per SIMD, so every load a batch
 // needs is issued a batch ahead, into the registers the batch before has
-// given up.  32 rows of 512 slots, 61 updates of 512 tokens: 1724 us with the
+// given up.  32 rows of 512 slots, 61 updates of 512 tokens, a tenth of the
+// keys around eight centres (uneven lists: Gaussian keys take 1060): 1724 us with the
 // routes compacted in every wave and each batch's loads waited for, 1377 so
 // (plus 18 for k_route_sort), 1319 with the sums rounded to bf16 here (which
 // also takes two casts of dk / dv, 330 us, out of the training step).
